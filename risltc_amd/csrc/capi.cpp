@@ -1263,6 +1263,7 @@ static int upload_mesh(risltc_context_t* c, const uint32_t* positions, const uin
 static rl::BvhView bvh_view_of(const rl::BvhBuild& b) {
     rl::BvhView v;
     v.rec = b.rec;
+    v.wide = b.wide;
     v.units = b.units;
     v.leaf_count = b.leaf_count;
     return v;

@@ -62,11 +62,23 @@ struct SceneView {
 // first unit past the node's subtree). Leaf: 3 units (v0.xyz | -1,
 // v1.xyz | triangle id, v2.xyz | light flag bit 31); it continues at the next
 // record. Traversal ends at unit `units`; two zero units of padding follow.
+// The shadow walk reads the same boxes from four-way nodes of kWideFloat4
+// 16-byte words (64 bytes): a grid origin (3 floats) and its steps (3 floats),
+// then per axis the low and the high planes of the four slots in bytes (plane =
+// origin + byte * step), then their references (>= 0: a wide node, node 0 the
+// root; < 0: a triangle record or a pair of them in rec). The words are
+// origin x y z, step x | step y z, low x, high x | low y, high y, low z,
+// high z | references.
 struct BvhView {
     const float4* rec;
+    const float4* wide;   // null: no wide nodes
     uint32_t units;       // 5 * leaf_count - 2
     uint32_t leaf_count;
 };
+constexpr uint32_t kWideFloat4 = 4;
+// units that a leaf reference can address beside its pair bit
+constexpr uint64_t kMaxWideUnits = 1ull << 30;
+constexpr uint32_t kWideLevels = 63;
 // largest triangle count whose pre-order units fit a signed 32-bit index
 constexpr uint64_t kMaxBvhTriangles = 400000000ull;
 
@@ -241,9 +253,9 @@ struct ShadeArgs {
 };
 
 // The shadow-ray list is cut into kTraceQueues equal slices, one per XCD:
-// work-group b runs on XCD b mod 8, starts on slice b mod 8 and takes rays
-// from that slice's counter (queues[kQueueStride * q]) until it is empty,
-// then moves on to the next slice. The counters start at zero.
+// work-group b runs on XCD b mod 8, starts on slice b mod 8 and takes runs of
+// rays from that slice (the first by its place, then from the slice's counter
+// queues[kQueueStride * q]) until it is empty, then moves on to the next. The counters start at zero.
 constexpr uint32_t kTraceQueues = 8;
 constexpr uint32_t kQueueStride = 32;  // words: one 128-byte line per counter
 
@@ -259,7 +271,7 @@ struct TraceArgs {
     uint32_t max_rays;
     uint32_t* hits;     // one word per slot
     uint32_t* queues;   // kTraceQueues * kQueueStride words, zeroed
-    uint32_t refill;    // a wave fetches rays once this many lanes are idle
+    uint32_t refill;    // a wave fetches rays once half this many lanes are idle
 };
 
 struct ResolveArgs {
@@ -325,6 +337,7 @@ hipError_t launch_fill_u32(uint32_t* p, uint32_t n, uint32_t v, hipStream_t s);
 
 struct BvhBuild {
     float4* rec = nullptr;
+    float4* wide = nullptr;
     uint32_t units = 0;
     uint32_t leaf_count = 0;
 };
