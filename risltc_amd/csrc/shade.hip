@@ -161,20 +161,14 @@ __device__ __forceinline__ float edge_term(f3 a, f3 b) {
 // contributes its clipped part; the closing edge exit -> entry is added last.
 // The exact build sums the terms in the order of the reference's rotated
 // output (c_clip_rot), the fast build in input-edge order.
+// This is the general form; mask: the input vertices above the horizon, not 0.
 template <bool X>
-__device__ __forceinline__ float polygon_ltc(const float* px, const float* py, const float* pz, uint32_t n,
-                                             uint32_t& vc) {
+__device__ __forceinline__ float polygon_ltc_clipped(const float* px, const float* py, const float* pz, uint32_t n,
+                                                     uint32_t mask) {
     const uint32_t full = (1u << n) - 1u;
-    uint32_t mask = 0;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) mask |= (pz[i] > 0.0f) ? (1u << i) : 0u;
-    mask &= full;
-    vc = 0;
-    if (mask == 0) return 0.0f;
-    uint32_t k = __builtin_popcount(mask);
-    bool clipped = mask != full;
-    uint32_t L = clipped ? k + 2u : n;
-    vc = L;
+    const uint32_t k = __builtin_popcount(mask);
+    const bool clipped = mask != full;
+    const uint32_t L = clipped ? k + 2u : n;
     // slots n..8 of px/py/pz hold vertex 0 (the light records repeat it), so
     // edge i always ends at slot i + 1: static indices, no address selects
     f3 nv[9];
@@ -246,6 +240,55 @@ __device__ __forceinline__ float polygon_ltc(const float* px, const float* py, c
             if ((uint32_t)i < L) acc += t[i];
     }
     return fabs_(acc);
+}
+
+// The clipped polygon's LTC integral; vc: its vertex count (0: below the
+// horizon).
+// The candidate evaluation is bound by VALU issue, and this is most of it. On
+// the 1080p city 0.8% of the polygons are clipped, so of a wave's 64 about six
+// waves in ten have none; their edges need no horizon points, no choice of
+// end points and (rarely long) no reciprocal square root. The fast build runs
+// those waves through straight-line code with the same operations per edge in
+// the same order: 22 instead of 37 VALU instructions per edge and no branches
+// (shade kernel, 1080p city: 3.80 -> 3.37 ms; learned pass 6.7 -> 5.8).
+template <bool X>
+__device__ __forceinline__ float polygon_ltc(const float* px, const float* py, const float* pz, uint32_t n,
+                                             uint32_t& vc) {
+    const uint32_t full = (1u << n) - 1u;
+    uint32_t mask = 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) mask |= (pz[i] > 0.0f) ? (1u << i) : 0u;
+    mask &= full;
+    const bool clipped = mask != full;
+    vc = mask == 0u ? 0u : (clipped ? (uint32_t)__builtin_popcount(mask) + 2u : n);
+    float r = 0.0f;
+    bool general = X || __builtin_amdgcn_ballot_w64(clipped && mask != 0u) != 0ull;
+    if constexpr (!X) {
+        if (!general) {
+            const f3 first = normalize3<false>(mk3(px[0], py[0], pz[0]));
+            f3 a = first;
+            float acc = 0.0f, shortest = 1.0f;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const f3 b = i == 7 ? first : normalize3<false>(mk3(px[i + 1], py[i + 1], pz[i + 1]));
+                const float x = dot3(a, b), y = fabs_(x);
+                const float A = fma_(fma_(0.0145206f, y, 0.4965155f), y, 0.8543985f);
+                const float B = fma_(y + 4.1616724f, y, 3.4175940f);
+                const float term = fma_(a.x, b.y, -(a.y * b.x)) * div_<false>(A, B);
+                // (slots n..8 hold vertex 0: edge n - 1 closes the polygon)
+                acc = (uint32_t)i < n ? acc + term : acc;
+                shortest = fmin_(shortest, x);
+                a = b;
+            }
+            r = mask != 0u ? fabs_(acc) : 0.0f;
+            // an edge longer than 90 degrees (or a NaN) takes the general form
+            general = __builtin_amdgcn_ballot_w64(mask != 0u && !(shortest > 0.0f)) != 0ull;
+        }
+    }
+    if (general) {
+        if (mask != 0u) r = polygon_ltc_clipped<X>(px, py, pz, n, mask);
+    }
+    return r;
 }
 
 // ---- clipped polygon, materialised in the reference's output order --------
