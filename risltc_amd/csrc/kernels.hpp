@@ -345,10 +345,10 @@ struct BvhBuild {
 // nodes, node 0 the root. Leaves have left = right = -1 and prim = triangle;
 // count = triangles below a node; box = 6 floats (internal nodes).
 struct SahTree {
-    float* tbox;    // 6 per triangle (lo xyz, hi xyz)
+    float* tbox;    // 6 per triangle (lo xyz, hi xyz; order-preserving integer images)
     float* cent;    // 3 per triangle
     uint32_t* idx;  // triangle permutation, partitioned in place
-    uint32_t* tmp;  // partition buffer
+    uint32_t* tmp;  // its other half: levels alternate between the two
     int* left;
     int* right;
     int* parent;
@@ -358,7 +358,8 @@ struct SahTree {
     float* box;
     uint32_t* node_counter;
 };
-hipError_t build_sah_tree(const float* tris, uint32_t n, SahTree& T, hipStream_t s);
+size_t sah_scratch_bytes(uint32_t n);
+hipError_t build_sah_tree(const float* tris, uint32_t n, SahTree& T, void* scratch, hipStream_t s);
 // Builds the hierarchy (RISLTC_BVH_SAH or RISLTC_BVH_LBVH) of the dequantised
 // triangles of a *.vks mesh on the device and lays it out in pre-order.
 hipError_t build_bvh(const uint2* d_positions, uint64_t triangle_count, const float deq_factor[3],

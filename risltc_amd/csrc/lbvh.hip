@@ -400,19 +400,19 @@ __global__ void fill_u32(uint32_t* p, uint64_t n, uint32_t v) {
 }
 
 namespace {
-// device allocations of one build, released on every path
+// The device memory of one build: one allocation, released on every path
+// (twenty cost a millisecond). Carved twice: without memory to measure it,
+// then for the pointers.
 struct BuildScratch {
-    void* p[20] = {};
-    int k = 0;
+    char* base = nullptr;
+    size_t used = 0;
     template <class T>
-    hipError_t get(T** out, size_t bytes) {
-        *out = nullptr;
-        hipError_t e = hipMalloc((void**)out, bytes);
-        if (e == hipSuccess) p[k++] = *out;
-        return e;
+    void get(T** out, size_t bytes) {
+        *out = base ? reinterpret_cast<T*>(base + used) : nullptr;
+        used += (bytes + 255u) & ~(size_t)255u;
     }
     ~BuildScratch() {
-        for (int i = 0; i < k; ++i) hipFree(p[i]);
+        if (base) hipFree(base);
     }
 };
 }  // namespace
@@ -470,34 +470,60 @@ hipError_t build_bvh(const uint2* d_pos, uint64_t tri_count, const float deq_fac
                      uint32_t builder, BvhBuild* out, hipStream_t s) {
     if (tri_count == 0 || tri_count > kMaxBvhTriangles) return hipErrorInvalidValue;
     if (builder != RISLTC_BVH_SAH && builder != RISLTC_BVH_LBVH) return hipErrorInvalidValue;
-    BuildScratch w;
     const int n = (int)tri_count;
     const uint64_t nodes = 2 * tri_count - 1;
     const uint32_t tb = 256;
     const uint32_t tri_blocks = (uint32_t)((tri_count + tb - 1) / tb);
     const uint32_t node_blocks = (uint32_t)((nodes + tb - 1) / tb);
-    float *tris, *cent, *box;
+    const uint32_t red_blocks = 1024;
+    const bool sah = builder == RISLTC_BVH_SAH;
+    float *tris, *cent, *box, *partial, *bounds;
     int *left, *right, *parent, *count;
-    uint32_t* prim;
-    // (the layout keeps its units in the centroids' space, and the wide nodes'
-    // scratch follows in the triangles' space)
-    BVH_TRY(w.get(&tris, std::max(sizeof(float) * 9 * tri_count, wide_scratch_bytes((uint32_t)n))));
-    BVH_TRY(w.get(&cent, sizeof(float) * 3 * tri_count));
+    uint32_t *prim, *arrivals;
+    uint64_t *keys, *keys_sorted;
+    void *temp, *sah_scratch;
+    size_t temp_bytes = 0;
+    SahTree T;
+    if (!sah)
+        BVH_TRY(hipcub::DeviceRadixSort::SortKeys(nullptr, temp_bytes, (uint64_t*)nullptr, (uint64_t*)nullptr, n, 0, 64, s));
+    auto carve = [&](BuildScratch& w) {
+        // (the layout keeps its units in the centroids' space, and the wide
+        // nodes' scratch follows in the triangles' space)
+        w.get(&tris, std::max(sizeof(float) * 9 * tri_count, wide_scratch_bytes((uint32_t)n)));
+        w.get(&cent, sizeof(float) * 3 * tri_count);
+        w.get(&box, sizeof(float) * 6 * nodes);
+        w.get(&left, sizeof(int) * nodes);
+        w.get(&right, sizeof(int) * nodes);
+        w.get(&parent, sizeof(int) * nodes);
+        w.get(&count, sizeof(int) * nodes);
+        w.get(&prim, sizeof(uint32_t) * nodes);
+        if (sah) {
+            w.get(&T.tbox, sizeof(float) * 6 * tri_count);
+            w.get(&T.idx, sizeof(uint32_t) * tri_count);
+            w.get(&T.tmp, sizeof(uint32_t) * tri_count);
+            w.get(&T.first, sizeof(int) * nodes);
+            w.get(&T.node_counter, sizeof(uint32_t));
+            w.get(&sah_scratch, sah_scratch_bytes((uint32_t)n));
+        } else {
+            w.get(&partial, sizeof(float) * 6 * red_blocks);
+            w.get(&bounds, sizeof(float) * 6);
+            w.get(&keys, sizeof(uint64_t) * tri_count);
+            w.get(&keys_sorted, sizeof(uint64_t) * tri_count);
+            w.get(&arrivals, sizeof(uint32_t) * tri_count);
+            w.get(&temp, temp_bytes);
+        }
+    };
+    BuildScratch w;
+    carve(w);
+    BVH_TRY(hipMalloc(&w.base, w.used));
+    w.used = 0;
+    carve(w);
     int* unit = reinterpret_cast<int*>(cent);
-    BVH_TRY(w.get(&box, sizeof(float) * 6 * nodes));
-    BVH_TRY(w.get(&left, sizeof(int) * nodes));
-    BVH_TRY(w.get(&right, sizeof(int) * nodes));
-    BVH_TRY(w.get(&parent, sizeof(int) * nodes));
-    BVH_TRY(w.get(&count, sizeof(int) * nodes));
-    BVH_TRY(w.get(&prim, sizeof(uint32_t) * nodes));
     hipLaunchKernelGGL(dequant_kernel, dim3(tri_blocks), dim3(tb), 0, s, d_pos, tri_count,
                        make_float3(deq_factor[0], deq_factor[1], deq_factor[2]),
                        make_float3(deq_summand[0], deq_summand[1], deq_summand[2]), tris, cent);
-    hipLaunchKernelGGL(fill_u32, dim3(node_blocks), dim3(tb), 0, s, reinterpret_cast<uint32_t*>(parent), nodes,
-                       0xFFFFFFFFu);
     BVH_TRY(hipGetLastError());
-    if (builder == RISLTC_BVH_SAH) {
-        SahTree T;
+    if (sah) {
         T.cent = cent;
         T.left = left;
         T.right = right;
@@ -505,30 +531,15 @@ hipError_t build_bvh(const uint2* d_pos, uint64_t tri_count, const float deq_fac
         T.count = count;
         T.prim = prim;
         T.box = box;
-        BVH_TRY(w.get(&T.tbox, sizeof(float) * 6 * tri_count));
-        BVH_TRY(w.get(&T.idx, sizeof(uint32_t) * tri_count));
-        BVH_TRY(w.get(&T.tmp, sizeof(uint32_t) * tri_count));
-        BVH_TRY(w.get(&T.first, sizeof(int) * nodes));
-        BVH_TRY(w.get(&T.node_counter, sizeof(uint32_t)));
-        BVH_TRY(build_sah_tree(tris, (uint32_t)n, T, s));
+        BVH_TRY(build_sah_tree(tris, (uint32_t)n, T, sah_scratch, s));
     } else {
-        const uint32_t red_blocks = 1024;
-        float *partial, *bounds;
-        uint64_t *keys, *keys_sorted;
-        uint32_t* arrivals;
-        void* temp;
-        size_t temp_bytes = 0;
-        BVH_TRY(w.get(&partial, sizeof(float) * 6 * red_blocks));
-        BVH_TRY(w.get(&bounds, sizeof(float) * 6));
-        BVH_TRY(w.get(&keys, sizeof(uint64_t) * tri_count));
-        BVH_TRY(w.get(&keys_sorted, sizeof(uint64_t) * tri_count));
-        BVH_TRY(w.get(&arrivals, sizeof(uint32_t) * tri_count));
+        // (the root keeps no parent)
+        hipLaunchKernelGGL(fill_u32, dim3(node_blocks), dim3(tb), 0, s, reinterpret_cast<uint32_t*>(parent), nodes,
+                           0xFFFFFFFFu);
         hipLaunchKernelGGL(bounds_kernel, dim3(red_blocks), dim3(256), 0, s, cent, tri_count, partial);
         hipLaunchKernelGGL(bounds_final_kernel, dim3(1), dim3(64), 0, s, partial, red_blocks, bounds);
         hipLaunchKernelGGL(morton_kernel, dim3(tri_blocks), dim3(tb), 0, s, cent, tri_count, bounds, keys);
         BVH_TRY(hipGetLastError());
-        BVH_TRY(hipcub::DeviceRadixSort::SortKeys(nullptr, temp_bytes, keys, keys_sorted, n, 0, 64, s));
-        BVH_TRY(w.get(&temp, temp_bytes));
         BVH_TRY(hipcub::DeviceRadixSort::SortKeys(temp, temp_bytes, keys, keys_sorted, n, 0, 64, s));
         hipLaunchKernelGGL(fill_u32, dim3(tri_blocks), dim3(tb), 0, s, arrivals, tri_count, 0u);
         if (n > 1)
