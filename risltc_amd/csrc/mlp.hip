@@ -528,72 +528,16 @@ hipError_t launch_proposal(const ProposalArgs& a, hipStream_t s) {
 }
 
 // ---- training --------------------------------------------------------------------
-// C[M][N] = A[M][K] . Bt[N][K]^T, bf16 operands, FP32 accumulation. One wave
-// computes a 16 x 32 block; gridDim.z splits K into slices of kslice.
-enum GemmEpilogue { kEpiHidden = 0, kEpiLogits = 1, kEpiBackward = 2, kEpiPartial = 3 };
-
-struct GemmArgs {
-    const uint16_t* A;
-    const uint16_t* Bt;
-    uint32_t M, N, K, lda, ldb, kslice;
-    const float* bias;      // hidden, logits
-    uint16_t* out;          // hidden, backward: [M][N] bf16
-    uint16_t* out_t;        // hidden, backward: [N][M] bf16
-    float* outf;            // logits: [M][N]; partial: [slice][M][N]
-    const uint16_t* mask;   // backward: [M][N] bf16 activation (relu mask)
-};
-
-template <int EPI>
-__global__ void __launch_bounds__(256) gemm_nt_kernel(GemmArgs g) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int gq = lane >> 4, r = lane & 15;
-    const uint32_t nblk = g.N / 32u;
-    const uint32_t blk = blockIdx.x * 4u + (uint32_t)wave;
-    if (blk >= (g.M / 16u) * nblk) return;
-    const uint32_t m0 = (blk / nblk) * 16u, n0 = (blk % nblk) * 32u;
-    const uint32_t k0 = blockIdx.z * g.kslice, k1 = min(g.K, k0 + g.kslice);
-    f32x4 acc0 = {0.0f, 0.0f, 0.0f, 0.0f}, acc1 = acc0;
-    for (uint32_t k = k0; k < k1; k += 32u) {
-        bf16x8 a = frag(g.A + (size_t)(m0 + r) * g.lda + k + 8 * gq);
-        acc0 = mfma(a, frag(g.Bt + (size_t)(n0 + r) * g.ldb + k + 8 * gq), acc0);
-        acc1 = mfma(a, frag(g.Bt + (size_t)(n0 + 16 + r) * g.ldb + k + 8 * gq), acc1);
-    }
-    // acc_t[i] = C[m0 + 4 gq + i][n0 + 16 t + r]
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-        const f32x4 acc = t ? acc1 : acc0;
-        const uint32_t n = n0 + 16u * t + (uint32_t)r;
-        uint32_t packed[2] = {0u, 0u};
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const uint32_t m = m0 + 4u * gq + i;
-            float v = acc[i];
-            if constexpr (EPI == kEpiHidden) {
-                v = fmax_(v + g.bias[n], 0.0f);
-            } else if constexpr (EPI == kEpiLogits) {
-                g.outf[(size_t)m * g.N + n] = v + g.bias[n];
-            } else if constexpr (EPI == kEpiBackward) {
-                if (!(bf16_float(g.mask[(size_t)m * g.N + n]) > 0.0f)) v = 0.0f;
-            } else {
-                g.outf[((size_t)blockIdx.z * g.M + m) * g.N + n] = v;
-            }
-            if constexpr (EPI == kEpiHidden || EPI == kEpiBackward) {
-                uint16_t b = bf16_bits(v);
-                g.out[(size_t)m * g.N + n] = b;
-                packed[i >> 1] |= (uint32_t)b << (16 * (i & 1));
-            }
-        }
-        if constexpr (EPI == kEpiHidden || EPI == kEpiBackward)
-            *reinterpret_cast<uint2*>(g.out_t + (size_t)n * g.M + m0 + 4u * gq) = make_uint2(packed[0], packed[1]);
-    }
-}
-
-template <int EPI>
-static void gemm(const GemmArgs& g, uint32_t slices, hipStream_t s) {
-    uint32_t blocks = ((g.M / 16u) * (g.N / 32u) + 3u) / 4u;
-    hipLaunchKernelGGL(gemm_nt_kernel<EPI>, dim3(blocks, 1, slices), dim3(256), 0, s, g);
-}
-
+// A step is four kernels: the batch's features (train_gather_kernel), the
+// forward and backward pass of the batch's rows (train_rows_kernel), the
+// weight gradients as split-K products (weight_grad_kernel) and their
+// reduction with the Adam update (train_finish_kernel). The rows are
+// independent until the weight gradients, so a work-group keeps its rows'
+// activations and logits in LDS; what leaves it are the transposed
+// activations and gradients, whose rows the weight gradients read K-contiguous.
+// What bounds it: 12 GFLOP on 65,536 rows are 10 us of matrix cores; the 24
+// small launches that this replaces took 830 us (of them 440 in sums by one
+// work-group with one load in flight).
 __device__ __forceinline__ uint32_t hash32(uint32_t x) {
     x ^= x >> 16;
     x *= 0x7feb352du;
@@ -604,10 +548,11 @@ __device__ __forceinline__ uint32_t hash32(uint32_t x) {
 }
 
 // batch item b: a pseudo-random pixel-sample; features (both layouts), the
-// cluster of its selected light and a weight (1, or 0 without a selection)
-__global__ void train_gather_kernel(TrainArgs A, uint16_t* X, uint16_t* Xt, uint32_t* target, float* y) {
+// cluster of its selected light and a weight (1, or 0 without a selection);
+// count: the items of weight 1
+__global__ void __launch_bounds__(256) train_gather_kernel(TrainArgs A, uint16_t* X, uint16_t* Xt, uint32_t* target,
+                                                           float* y, uint32_t* count) {
     const uint32_t b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= A.B) return;
     const uint32_t item = hash32(A.seed * 0x9E3779B9u + b) % A.sample_count;
     const uint32_t pixel = item / A.spp;
     float f[kMlpIn];
@@ -620,33 +565,17 @@ __global__ void train_gather_kernel(TrainArgs A, uint16_t* X, uint16_t* Xt, uint
     }
     target[b] = c;
     y[b] = w;
-    for (int k = 0; k < kMlpIn; ++k) {
-        uint16_t h = bf16_bits(f[k]);
-        X[(size_t)b * kMlpIn + k] = h;
-        Xt[(size_t)k * A.B + b] = h;
-    }
+    const uint32_t used = (uint32_t)__popcll(__ballot(w != 0.0f));
+    if ((threadIdx.x & 63u) == 0u && used != 0u) atomicAdd(count, used);
+    uint32_t p[kMlpIn / 2];
+#pragma unroll
+    for (int k = 0; k < kMlpIn / 2; ++k) p[k] = bf16_pack2(f[2 * k], f[2 * k + 1]);
+    uint4* row = reinterpret_cast<uint4*>(X + (size_t)b * kMlpIn);
+#pragma unroll
+    for (int k = 0; k < kMlpIn / 8; ++k) row[k] = make_uint4(p[4 * k], p[4 * k + 1], p[4 * k + 2], p[4 * k + 3]);
+#pragma unroll
+    for (int k = 0; k < kMlpIn; ++k) Xt[(size_t)k * A.B + b] = (uint16_t)(p[k / 2] >> (16 * (k & 1)));
 }
-
-// sum of y over the batch in a fixed order (one block)
-__global__ void batch_sum_kernel(const float* y, uint32_t B, float* out) {
-    __shared__ float part[256];
-    float s = 0.0f;
-    for (uint32_t i = threadIdx.x; i < B; i += 256u) s += y[i];
-    part[threadIdx.x] = s;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) part[threadIdx.x] += part[threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) *out = part[0];
-}
-
-// dL/dz = (y_b / Y) (softmax(z_b) - onehot(c_b)); per-row loss terms. A
-// work-group takes ROWS rows, one wave per row at a time (each lane OUT / 64
-// of the logits, coalesced), and writes the transposed gradient Gt through
-// LDS so that each thread stores whole 16-byte pieces of its columns.
-template <int OUT>
-constexpr int sg_rows() { return OUT > 256 ? 16 : 64; }
 
 __device__ __forceinline__ float wave_max(float v) {
 #pragma unroll
@@ -659,21 +588,116 @@ __device__ __forceinline__ float wave_sum(float v) {
     return v;
 }
 
+// rows per work-group: their logits fill 32 to 64 KB of LDS; 8 waves (with 4,
+// the default network's 65,536 rows take 85 us instead of 66)
+constexpr int kRowWaves = 8;
 template <int OUT>
-__global__ void __launch_bounds__(256) softmax_grad_kernel(const float* Z, const uint32_t* target, const float* y,
-                                                           const float* ysum, uint32_t B, uint16_t* G, uint16_t* Gt,
-                                                           float* row_loss) {
-    constexpr int ROWS = sg_rows<OUT>(), PER = OUT / 64, LD = OUT + 8;
-    __shared__ uint16_t tile[ROWS * LD];
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+constexpr int train_rows() { return OUT > 256 ? 16 : 32; }
+
+template <int HID, int OUT>
+struct RowsShared {
+    static constexpr int kRows = train_rows<OUT>();
+    static constexpr int kLdZ = OUT + 4;      // floats per row of logits
+    static constexpr int kLdG = 2 * kLdZ;     // the same row's gradient as bf16, in place
+    uint16_t x[kRows * kLdW1];
+    uint16_t h[3][kRows * ld_h<HID>()];
+    uint16_t g[2][kRows * ld_h<HID>()];
+    float z[kRows * kLdZ];
+};
+static_assert(sizeof(RowsShared<64, 256>) <= 80 * 1024, "two work-groups per CU");
+static_assert(sizeof(RowsShared<128, 1024>) <= 160 * 1024, "LDS");
+
+// C[m][n] = A[m][K] . Wt[n][K]^T of the work-group's rows, A in LDS, Wt in
+// global memory (it stays in L2): put(m, n, four values of rows m..m + 3)
+template <int ROWS, int N, int K, int LDA, class F>
+__device__ __forceinline__ void rows_product(const uint16_t* A, const uint16_t* Wt, F put) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, gq = lane >> 4, r = lane & 15;
+    // (a wave keeps its rows, so that narrow layers occupy every wave)
+    constexpr int MT = ROWS / 16, WN = kRowWaves / MT;
+    const int m = wave / WN;
+    for (int t = wave % WN; t < N / 16; t += WN) {
+        bf16x8 b[K / 32];
+#pragma unroll
+        for (int k = 0; k < K / 32; ++k) b[k] = frag(Wt + (size_t)(16 * t + r) * K + 32 * k + 8 * gq);
+        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int k = 0; k < K / 32; ++k) acc = mfma(frag(A + (16 * m + r) * LDA + 32 * k + 8 * gq), b[k], acc);
+        put(16 * m + 4 * gq, 16 * t + r, acc);
+    }
+}
+
+// dst[n][b0 ..] = column n of the work-group's rows (LDS, LD values a row)
+template <int ROWS, int N, int LD>
+__device__ __forceinline__ void put_transposed(const uint16_t* src, uint16_t* dst, uint32_t B, uint32_t b0) {
+    for (int e = threadIdx.x; e < N * (ROWS / 8); e += 64 * kRowWaves) {
+        const int n = e % N, q = 8 * (e / N);
+        uint32_t w[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            w[j] = (uint32_t)src[(q + 2 * j) * LD + n] | ((uint32_t)src[(q + 2 * j + 1) * LD + n] << 16);
+        *reinterpret_cast<uint4*>(dst + (size_t)n * B + b0 + q) = make_uint4(w[0], w[1], w[2], w[3]);
+    }
+}
+
+struct RowsArgs {
+    MlpLayout L;
+    const uint16_t *wf, *wb;
+    const float* params;
+    const uint16_t* X;
+    const uint32_t* target;
+    const float* y;
+    const uint32_t* count;
+    uint32_t B;
+    uint16_t *Ht[3], *Gt[4];  // Gt[l]: gradient at the output of layer l + 1
+    float* row_loss;
+};
+
+template <int HID, int OUT>
+__global__ void __launch_bounds__(64 * kRowWaves) train_rows_kernel(RowsArgs A) {
+    constexpr int ROWS = train_rows<OUT>(), LDH = ld_h<HID>(), PER = OUT / 64;
+    using Sh = RowsShared<HID, OUT>;
+    constexpr MlpLayout L = mlp_layout(HID, OUT);
+    __shared__ Sh sh;
     const uint32_t b0 = blockIdx.x * ROWS;  // B is a multiple of ROWS
-    const float Y = *ysum;
-    for (uint32_t rr = 0; rr < ROWS / 4; ++rr) {
-        const uint32_t r = wave * (ROWS / 4) + rr, b = b0 + r;
-        const float* z = Z + (size_t)b * OUT;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    for (int e = threadIdx.x; e < ROWS * (kMlpIn / 8); e += 64 * kRowWaves) {
+        const int row = e / (kMlpIn / 8), q = e % (kMlpIn / 8);
+        *reinterpret_cast<uint4*>(sh.x + row * kLdW1 + 8 * q) =
+            *reinterpret_cast<const uint4*>(A.X + (size_t)(b0 + row) * kMlpIn + 8 * q);
+    }
+    __syncthreads();
+    // forward
+    auto hidden = [&](int layer, int bias) {
+        return [&A, layer, bias](int m, int n, f32x4 v) {
+            const float c = A.params[bias + n];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) sh.h[layer][(m + i) * LDH + n] = bf16_bits(fmax_(v[i] + c, 0.0f));
+        };
+    };
+    rows_product<ROWS, HID, kMlpIn, kLdW1>(sh.x, A.wf + L.pw1, hidden(0, L.pb1));
+    __syncthreads();
+    rows_product<ROWS, HID, HID, LDH>(sh.h[0], A.wf + L.pw2, hidden(1, L.pb2));
+    __syncthreads();
+    rows_product<ROWS, HID, HID, LDH>(sh.h[1], A.wf + L.pw3, hidden(2, L.pb3));
+    __syncthreads();
+    rows_product<ROWS, OUT, HID, LDH>(sh.h[2], A.wf + L.pw4, [&](int m, int n, f32x4 v) {
+        const float c = A.params[L.pb4 + n];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sh.z[(m + i) * Sh::kLdZ + n] = v[i] + c;
+    });
+#pragma unroll
+    for (int l = 0; l < 3; ++l) put_transposed<ROWS, HID, LDH>(sh.h[l], A.Ht[l], A.B, b0);
+    __syncthreads();
+    // dL/dz = (y_b / Y) (softmax(z_b) - onehot(c_b)), one wave per row at a
+    // time, each lane OUT / 64 of the logits; the row's loss term
+    uint16_t* g4 = reinterpret_cast<uint16_t*>(sh.z);
+    const float Y = (float)*A.count;
+    for (int rr = 0; rr < ROWS / kRowWaves; ++rr) {
+        const int r = wave * (ROWS / kRowWaves) + rr;
+        const uint32_t b = b0 + r;
         float v[PER];
 #pragma unroll
-        for (int k = 0; k < PER; ++k) v[k] = z[lane + 64u * k];
+        for (int k = 0; k < PER; ++k) v[k] = sh.z[r * Sh::kLdZ + lane + 64 * k];
         float m = v[0];
 #pragma unroll
         for (int k = 1; k < PER; ++k) m = fmax_(m, v[k]);
@@ -685,15 +709,13 @@ __global__ void __launch_bounds__(256) softmax_grad_kernel(const float* Z, const
             part += e[k];
         }
         const float s = wave_sum(part);
-        const float wb = Y > 0.0f ? y[b] / Y : 0.0f;
-        const uint32_t c = target[b];
+        const float wb = Y > 0.0f ? A.y[b] / Y : 0.0f;
+        const uint32_t c = A.target[b];
+        wave_sync();
 #pragma unroll
         for (int k = 0; k < PER; ++k) {
-            const uint32_t n = lane + 64u * k;
-            float d = wb * (e[k] / s - (n == c ? 1.0f : 0.0f));
-            uint16_t h = bf16_bits(d);
-            G[(size_t)b * OUT + n] = h;
-            tile[r * LD + n] = h;
+            const uint32_t n = (uint32_t)lane + 64u * k;
+            g4[r * Sh::kLdG + n] = bf16_bits(wb * (e[k] / s - (n == c ? 1.0f : 0.0f)));
         }
         // z[c] from the lane that holds it (c is the same for the whole wave)
         float vc = v[0];
@@ -701,57 +723,78 @@ __global__ void __launch_bounds__(256) softmax_grad_kernel(const float* Z, const
         for (int k = 1; k < PER; ++k)
             if ((c >> 6) == (uint32_t)k) vc = v[k];
         const float zc = __shfl(vc, (int)(c & 63u));
-        if (lane == 0) row_loss[b] = wb > 0.0f ? -wb * (zc - zm - __logf(s)) : 0.0f;
+        if (lane == 0) A.row_loss[b] = wb > 0.0f ? -wb * (zc - zm - __logf(s)) : 0.0f;
     }
     __syncthreads();
-    // Gt[n][b0 .. b0 + ROWS - 1], 8 rows per 16-byte store
-    for (uint32_t n = threadIdx.x; n < (uint32_t)OUT; n += blockDim.x) {
+    // backward: dA[b][i] = sum_o G[b][o] W[o][i], masked by the activation
+    // (wb holds the weights as [in][out])
+    auto back = [&](int to, int layer) {
+        return [to, layer](int m, int n, f32x4 v) {
 #pragma unroll
-        for (int q = 0; q < ROWS; q += 8) {
-            uint32_t w[4];
+            for (int i = 0; i < 4; ++i)
+                sh.g[to][(m + i) * LDH + n] =
+                    bf16_float(sh.h[layer][(m + i) * LDH + n]) > 0.0f ? bf16_bits(v[i]) : (uint16_t)0;
+        };
+    };
+    rows_product<ROWS, HID, OUT, Sh::kLdG>(g4, A.wb + L.pw4, back(0, 2));
+    put_transposed<ROWS, OUT, Sh::kLdG>(g4, A.Gt[3], A.B, b0);
+    __syncthreads();
+    rows_product<ROWS, HID, HID, LDH>(sh.g[0], A.wb + L.pw3, back(1, 1));
+    put_transposed<ROWS, HID, LDH>(sh.g[0], A.Gt[2], A.B, b0);
+    __syncthreads();
+    rows_product<ROWS, HID, HID, LDH>(sh.g[1], A.wb + L.pw2, back(0, 0));
+    put_transposed<ROWS, HID, LDH>(sh.g[1], A.Gt[1], A.B, b0);
+    __syncthreads();
+    put_transposed<ROWS, HID, LDH>(sh.g[0], A.Gt[0], A.B, b0);
+}
+
+// Weight gradients of the four layers: partial[slice][o][i] = sum over the
+// slice's batch items of Gt[o][b] At[i][b]. One wave computes a 16 x 32 block
+// of one slice; the loads of four steps are in flight together.
+constexpr uint32_t kTrainSlice = 2048;  // batch items per slice
+struct GradArgs {
+    const uint16_t *Gt[4], *At[4];
+    uint32_t nout[4], nin[4];
+    uint32_t block0[5];   // 16 x 32 blocks of the layers, prefix sums
+    size_t partial0[4];   // of each layer's partial sums
+    uint32_t B, slices;
+    float* partial;
+};
+
+__global__ void __launch_bounds__(256) weight_grad_kernel(GradArgs g) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, gq = lane >> 4, r = lane & 15;
+    const uint32_t blk = blockIdx.x * 4u + (uint32_t)wave, slice = blockIdx.y;
+    if (blk >= g.block0[4]) return;
+    int l = 0;
+    while (l < 3 && blk >= g.block0[l + 1]) ++l;
+    const uint32_t nblk = g.nin[l] / 32u, e = blk - g.block0[l];
+    const uint32_t m0 = (e / nblk) * 16u, n0 = (e % nblk) * 32u;
+    const uint32_t k0 = slice * kTrainSlice, k1 = min(g.B, k0 + kTrainSlice);
+    const uint16_t* pa = g.Gt[l] + (size_t)(m0 + r) * g.B + 8 * gq;
+    const uint16_t* pb = g.At[l] + (size_t)(n0 + r) * g.B + 8 * gq;
+    const uint16_t* pc = pb + (size_t)16 * g.B;
+    f32x4 acc0 = {0.0f, 0.0f, 0.0f, 0.0f}, acc1 = acc0;
+    // (B is a multiple of 256, so a slice is a multiple of 128)
+    for (uint32_t k = k0; k < k1; k += 128u) {
+        bf16x8 a[4], b[4], c[4];
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
-                w[j] = (uint32_t)tile[(q + 2 * j) * LD + n] | ((uint32_t)tile[(q + 2 * j + 1) * LD + n] << 16);
-            *reinterpret_cast<uint4*>(Gt + (size_t)n * B + b0 + q) = make_uint4(w[0], w[1], w[2], w[3]);
+        for (int u = 0; u < 4; ++u) {
+            a[u] = frag(pa + k + 32 * u);
+            b[u] = frag(pb + k + 32 * u);
+            c[u] = frag(pc + k + 32 * u);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            acc0 = mfma(a[u], b[u], acc0);
+            acc1 = mfma(a[u], c[u], acc1);
         }
     }
-}
-
-// grad[w] = sum over slices (fixed order); bias grads = column sums of G
-__global__ void reduce_grad_kernel(const float* partial, uint32_t slices, uint32_t count, float* dst) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= count) return;
-    float s = 0.0f;
-    for (uint32_t k = 0; k < slices; ++k) s += partial[(size_t)k * count + i];
-    dst[i] = s;
-}
-
-// one block per column n of Gt[N][B]: fixed-order tree sum
-__global__ void bias_grad_kernel(const uint16_t* Gt, uint32_t B, float* dst) {
-    __shared__ float part[256];
-    const uint32_t n = blockIdx.x;
-    float s = 0.0f;
-    for (uint32_t i = threadIdx.x; i < B; i += 256u) s += bf16_float(Gt[(size_t)n * B + i]);
-    part[threadIdx.x] = s;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) part[threadIdx.x] += part[threadIdx.x + w];
-        __syncthreads();
+    float* o = g.partial + g.partial0[l] + (size_t)slice * g.nout[l] * g.nin[l];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        o[(size_t)(m0 + 4u * gq + i) * g.nin[l] + n0 + r] = acc0[i];
+        o[(size_t)(m0 + 4u * gq + i) * g.nin[l] + n0 + 16u + r] = acc1[i];
     }
-    if (threadIdx.x == 0) dst[n] = part[0];
-}
-
-__global__ void loss_sum_kernel(const float* row_loss, uint32_t B, float* out) {
-    __shared__ float part[256];
-    float s = 0.0f;
-    for (uint32_t i = threadIdx.x; i < B; i += 256u) s += row_loss[i];
-    part[threadIdx.x] = s;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) part[threadIdx.x] += part[threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) *out = part[0];
 }
 
 // bf16 copies of layer weights: wf = master layout [out][in], wb = [in][out]
@@ -782,10 +825,9 @@ __device__ __forceinline__ void write_copies(const MlpLayout& L, int e, float v,
     }
 }
 
-__global__ void adam_kernel(TrainArgs A) {
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= A.L.params) return;
-    const float gr = A.grad[e];
+// one Adam step of parameter e with gradient gr
+__device__ __forceinline__ void adam(const TrainArgs& A, int e, float gr) {
+    A.grad[e] = gr;
     const float m = A.beta1 * A.m[e] + (1.0f - A.beta1) * gr;
     const float v = A.beta2 * A.v[e] + (1.0f - A.beta2) * gr * gr;
     A.m[e] = m;
@@ -795,6 +837,82 @@ __global__ void adam_kernel(TrainArgs A) {
     const float p = A.params[e] - A.lr * (m / bc1) / (__builtin_sqrtf(v / bc2) + A.eps);
     A.params[e] = p;
     write_copies(A.L, e, p, A.wf, A.wb);
+}
+
+// thread t's values t, t + 256, .. of a row of n (a multiple of 256) summed in
+// that order, 16 loads in flight, then a fixed tree over the work-group
+template <class F>
+__device__ __forceinline__ float row_sum(uint32_t n, F at) {
+    __shared__ float part[256];
+    const uint32_t t = threadIdx.x;
+    float s = 0.0f;
+    uint32_t i = t;
+    for (; i + 15u * 256u < n; i += 16u * 256u) {
+        float v[16];
+#pragma unroll
+        for (uint32_t u = 0; u < 16u; ++u) v[u] = at(i + 256u * u);
+#pragma unroll
+        for (uint32_t u = 0; u < 16u; ++u) s += v[u];
+    }
+    for (; i < n; i += 256u) s += at(i);
+    part[t] = s;
+    __syncthreads();
+    for (uint32_t w = 128u; w > 0u; w >>= 1) {
+        if (t < w) part[t] += part[t + w];
+        __syncthreads();
+    }
+    return part[0];
+}
+
+// The end of a step, by work-group: 256 weights (their slices' sum in slice
+// order), or one bias (the sum of its row of Gt), each with its Adam update,
+// or the loss.
+struct FinishArgs {
+    TrainArgs t;
+    const uint16_t* Gt[4];
+    uint32_t weights[4], biases[4];  // counts
+    int w0[4], b0[4];                // parameter offsets
+    uint32_t block0[5];              // weight work-groups of the layers, prefix sums
+    size_t partial0[4];
+    uint32_t slices;
+    const float* partial;
+    const float* row_loss;
+};
+
+__global__ void __launch_bounds__(256) train_finish_kernel(FinishArgs F) {
+    uint32_t blk = blockIdx.x;
+    if (blk < F.block0[4]) {
+        int l = 0;
+        while (l < 3 && blk >= F.block0[l + 1]) ++l;
+        const uint32_t i = (blk - F.block0[l]) * 256u + threadIdx.x;
+        if (i >= F.weights[l]) return;
+        const float* p = F.partial + F.partial0[l] + i;
+        const size_t step = F.weights[l];
+        float s = 0.0f;
+        uint32_t k = 0;
+        for (; k + 8u <= F.slices; k += 8u) {
+            float v[8];
+#pragma unroll
+            for (uint32_t u = 0; u < 8u; ++u) v[u] = p[(k + u) * step];
+#pragma unroll
+            for (uint32_t u = 0; u < 8u; ++u) s += v[u];
+        }
+        for (; k < F.slices; ++k) s += p[k * step];
+        adam(F.t, F.w0[l] + (int)i, s);
+        return;
+    }
+    blk -= F.block0[4];
+    for (int l = 0; l < 4; ++l) {
+        if (blk < F.biases[l]) {
+            const uint16_t* g = F.Gt[l] + (size_t)blk * F.t.B;
+            const float s = row_sum(F.t.B, [&](uint32_t i) { return bf16_float(g[i]); });
+            if (threadIdx.x == 0) adam(F.t, F.b0[l] + (int)blk, s);
+            return;
+        }
+        blk -= F.biases[l];
+    }
+    const float s = row_sum(F.t.B, [&](uint32_t i) { return F.row_loss[i]; });
+    if (threadIdx.x == 0) *F.t.loss = s;
 }
 
 __global__ void sync_kernel(MlpLayout L, const float* params, uint16_t* wf, uint16_t* wb) {
@@ -809,11 +927,11 @@ hipError_t launch_mlp_sync(const MlpLayout& L, const float* params, uint16_t* wf
 }
 
 namespace {
-constexpr uint32_t kTrainSlice = 2048;  // split-K slice of the weight-gradient products
 struct TrainScratch {
-    uint16_t *X, *Xt, *H1, *H1t, *H2, *H2t, *H3, *H3t, *G4, *G4t, *G3, *G3t, *G2, *G2t, *G1, *G1t;
-    float *Z, *y, *ysum, *row_loss, *partial;
-    uint32_t* target;
+    uint16_t *X, *Xt, *Ht[3], *Gt[4];
+    float *y, *row_loss, *partial;
+    uint32_t *target, *count;
+    size_t partial0[4];  // of each layer's partial weight gradients
 };
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 TrainScratch carve(void* base, uint32_t B, int hid, int out, size_t* total) {
@@ -827,27 +945,20 @@ TrainScratch carve(void* base, uint32_t B, int hid, int out, size_t* total) {
     };
     t.X = (uint16_t*)take(2ull * B * kMlpIn);
     t.Xt = (uint16_t*)take(2ull * B * kMlpIn);
-    t.H1 = (uint16_t*)take(2ull * B * hid);
-    t.H1t = (uint16_t*)take(2ull * B * hid);
-    t.H2 = (uint16_t*)take(2ull * B * hid);
-    t.H2t = (uint16_t*)take(2ull * B * hid);
-    t.H3 = (uint16_t*)take(2ull * B * hid);
-    t.H3t = (uint16_t*)take(2ull * B * hid);
-    t.G4 = (uint16_t*)take(2ull * B * out);
-    t.G4t = (uint16_t*)take(2ull * B * out);
-    t.G3 = (uint16_t*)take(2ull * B * hid);
-    t.G3t = (uint16_t*)take(2ull * B * hid);
-    t.G2 = (uint16_t*)take(2ull * B * hid);
-    t.G2t = (uint16_t*)take(2ull * B * hid);
-    t.G1 = (uint16_t*)take(2ull * B * hid);
-    t.G1t = (uint16_t*)take(2ull * B * hid);
-    t.Z = (float*)take(4ull * B * out);
+    for (int l = 0; l < 3; ++l) t.Ht[l] = (uint16_t*)take(2ull * B * hid);
+    for (int l = 0; l < 4; ++l) t.Gt[l] = (uint16_t*)take(2ull * B * (l == 3 ? out : hid));
     t.y = (float*)take(4ull * B);
-    t.ysum = (float*)take(4);
     t.row_loss = (float*)take(4ull * B);
-    const uint32_t slices = (B + kTrainSlice - 1) / kTrainSlice;
-    t.partial = (float*)take(4ull * slices * out * hid);
+    const size_t slices = (B + kTrainSlice - 1) / kTrainSlice;
+    size_t sums = 0;
+    const size_t weights[4] = {(size_t)hid * kMlpIn, (size_t)hid * hid, (size_t)hid * hid, (size_t)out * hid};
+    for (int l = 0; l < 4; ++l) {
+        t.partial0[l] = sums;
+        sums += slices * weights[l];
+    }
+    t.partial = (float*)take(4ull * sums);
     t.target = (uint32_t*)take(4ull * B);
+    t.count = (uint32_t*)take(4);
     if (total) *total = off;
     return t;
 }
@@ -861,58 +972,52 @@ size_t train_scratch_bytes(uint32_t B, int hid, int out) {
 
 hipError_t launch_train_step(const TrainArgs& a, hipStream_t s) {
     if (a.B == 0 || a.B % 256u != 0u || a.sample_count == 0) return hipErrorInvalidValue;
-    const MlpLayout& L4 = a.L;
-    const uint32_t H = (uint32_t)L4.hid;
-    TrainScratch t = carve(a.scratch, a.B, L4.hid, L4.out, nullptr);
-    const uint32_t O = (uint32_t)L4.out;
-    const uint32_t B = a.B, slices = (B + kTrainSlice - 1) / kTrainSlice;
-    hipLaunchKernelGGL(train_gather_kernel, dim3(B / 256u), dim3(256), 0, s, a, t.X, t.Xt, t.target, t.y);
-    hipLaunchKernelGGL(batch_sum_kernel, dim3(1), dim3(256), 0, s, t.y, B, t.ysum);
-    // forward
-    GemmArgs g{};
-    g = GemmArgs{t.X, a.wf + L4.pw1, B, H, kMlpIn, kMlpIn, kMlpIn, kMlpIn, a.params + L4.pb1, t.H1, t.H1t, nullptr, nullptr};
-    gemm<kEpiHidden>(g, 1, s);
-    g = GemmArgs{t.H1, a.wf + L4.pw2, B, H, H, H, H, H, a.params + L4.pb2, t.H2, t.H2t, nullptr, nullptr};
-    gemm<kEpiHidden>(g, 1, s);
-    g = GemmArgs{t.H2, a.wf + L4.pw3, B, H, H, H, H, H, a.params + L4.pb3, t.H3, t.H3t, nullptr, nullptr};
-    gemm<kEpiHidden>(g, 1, s);
-    g = GemmArgs{t.H3, a.wf + L4.pw4, B, O, H, H, H, H, a.params + L4.pb4, nullptr, nullptr, t.Z, nullptr};
-    gemm<kEpiLogits>(g, 1, s);
-    if (O > 256u)
-        hipLaunchKernelGGL(softmax_grad_kernel<kMlpOutWide>, dim3(B / sg_rows<kMlpOutWide>()), dim3(256), 0, s, t.Z,
-                           t.target, t.y, t.ysum, B, t.G4, t.G4t, t.row_loss);
+    const MlpLayout& L = a.L;
+    const uint32_t H = (uint32_t)L.hid, O = (uint32_t)L.out, B = a.B, slices = (B + kTrainSlice - 1) / kTrainSlice;
+    if ((H != (uint32_t)kMlpHid && H != (uint32_t)kMlpHidWide) || (O != (uint32_t)kMlpOut && O != (uint32_t)kMlpOutWide))
+        return hipErrorInvalidValue;
+    const TrainScratch t = carve(a.scratch, B, L.hid, L.out, nullptr);
+    hipError_t e = launch_zero_u32(t.count, 1u, s);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(train_gather_kernel, dim3(B / 256u), dim3(256), 0, s, a, t.X, t.Xt, t.target, t.y, t.count);
+    RowsArgs r{L, a.wf, a.wb, a.params, t.X, t.target, t.y, t.count, B, {}, {}, t.row_loss};
+    for (int l = 0; l < 3; ++l) r.Ht[l] = t.Ht[l];
+    for (int l = 0; l < 4; ++l) r.Gt[l] = t.Gt[l];
+    const bool wide = H == (uint32_t)kMlpHidWide, many = O == (uint32_t)kMlpOutWide;
+    if (wide && many)
+        hipLaunchKernelGGL((train_rows_kernel<kMlpHidWide, kMlpOutWide>), dim3(B / 16u), dim3(64 * kRowWaves), 0, s, r);
+    else if (wide)
+        hipLaunchKernelGGL((train_rows_kernel<kMlpHidWide, kMlpOut>), dim3(B / 32u), dim3(64 * kRowWaves), 0, s, r);
+    else if (many)
+        hipLaunchKernelGGL((train_rows_kernel<kMlpHid, kMlpOutWide>), dim3(B / 16u), dim3(64 * kRowWaves), 0, s, r);
     else
-        hipLaunchKernelGGL(softmax_grad_kernel<kMlpOut>, dim3(B / sg_rows<kMlpOut>()), dim3(256), 0, s, t.Z, t.target,
-                           t.y, t.ysum, B, t.G4, t.G4t, t.row_loss);
-    hipLaunchKernelGGL(loss_sum_kernel, dim3(1), dim3(256), 0, s, t.row_loss, B, a.loss);
-    // layer 4: dW4[o][i] = sum_b G4[b][o] H3[b][i]; dH3 = G4 . W4, masked by H3 > 0
-    struct Layer {
-        const uint16_t *Gt, *At;
-        uint32_t nout, nin;
-        int w, bias;
-    };
-    const Layer layers[4] = {{t.G4t, t.H3t, O, H, L4.pw4, L4.pb4}, {t.G3t, t.H2t, H, H, L4.pw3, L4.pb3},
-                             {t.G2t, t.H1t, H, H, L4.pw2, L4.pb2}, {t.G1t, t.Xt, H, kMlpIn, L4.pw1, L4.pb1}};
-    const uint16_t* Gs[4] = {t.G4, t.G3, t.G2, t.G1};
-    uint16_t* Gn[4] = {t.G3, t.G2, t.G1, nullptr};
-    uint16_t* Gnt[4] = {t.G3t, t.G2t, t.G1t, nullptr};
-    const uint16_t* masks[4] = {t.H3, t.H2, t.H1, nullptr};
+        hipLaunchKernelGGL((train_rows_kernel<kMlpHid, kMlpOut>), dim3(B / 32u), dim3(64 * kRowWaves), 0, s, r);
+    GradArgs g{};
+    FinishArgs f{};
+    f.t = a;
+    const uint16_t* At[4] = {t.Xt, t.Ht[0], t.Ht[1], t.Ht[2]};
+    const int w0[4] = {L.pw1, L.pw2, L.pw3, L.pw4}, b0[4] = {L.pb1, L.pb2, L.pb3, L.pb4};
+    uint32_t biases = 0;
     for (int l = 0; l < 4; ++l) {
-        const Layer& L = layers[l];
-        g = GemmArgs{L.Gt, L.At, L.nout, L.nin, B, B, B, kTrainSlice, nullptr, nullptr, nullptr, t.partial, nullptr};
-        gemm<kEpiPartial>(g, slices, s);
-        const uint32_t cnt = L.nout * L.nin;
-        hipLaunchKernelGGL(reduce_grad_kernel, dim3((cnt + 255u) / 256u), dim3(256), 0, s, t.partial, slices, cnt,
-                           a.grad + L.w);
-        hipLaunchKernelGGL(bias_grad_kernel, dim3(L.nout), dim3(256), 0, s, L.Gt, B, a.grad + L.bias);
-        if (Gn[l]) {
-            // dA[b][i] = sum_o G[b][o] W[o][i]: Bt = W^T stored [in][out] = wb
-            g = GemmArgs{Gs[l], a.wb + L.w, B, L.nin, L.nout, L.nout, L.nout, L.nout, nullptr, Gn[l], Gnt[l], nullptr,
-                         masks[l]};
-            gemm<kEpiBackward>(g, 1, s);
-        }
+        g.Gt[l] = f.Gt[l] = t.Gt[l];
+        g.At[l] = At[l];
+        g.nout[l] = f.biases[l] = l == 3 ? O : H;
+        g.nin[l] = l == 0 ? (uint32_t)kMlpIn : H;
+        f.weights[l] = g.nout[l] * g.nin[l];
+        g.block0[l + 1] = g.block0[l] + f.weights[l] / (16u * 32u);
+        f.block0[l + 1] = f.block0[l] + (f.weights[l] + 255u) / 256u;
+        g.partial0[l] = f.partial0[l] = t.partial0[l];
+        f.w0[l] = w0[l];
+        f.b0[l] = b0[l];
+        biases += f.biases[l];
     }
-    hipLaunchKernelGGL(adam_kernel, dim3((L4.params + 255) / 256), dim3(256), 0, s, a);
+    g.B = B;
+    g.slices = f.slices = slices;
+    g.partial = t.partial;
+    f.partial = t.partial;
+    f.row_loss = t.row_loss;
+    hipLaunchKernelGGL(weight_grad_kernel, dim3((g.block0[4] + 3u) / 4u, slices), dim3(256), 0, s, g);
+    hipLaunchKernelGGL(train_finish_kernel, dim3(f.block0[4] + biases + 1u), dim3(256), 0, s, f);
     return hipGetLastError();
 }
 
