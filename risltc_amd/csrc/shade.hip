@@ -482,24 +482,34 @@ __device__ __forceinline__ void cas(Psa& P, int l, int r) {
 }
 
 // sort_convex_polygon_vertices (polygon_sampling.glsl:441-506); 9 vertices
-// (clipped 8-gons) use a complete 25-comparator network
+// (clipped 8-gons) use a complete 25-comparator network. A wave's lanes hold
+// every count, so branching on it runs all the networks one after the other:
+// 31 comparators for counts 3 to 8. The 19 below are a common
+// supersequence of those six (comparators on other vertices commute): each
+// lane takes its own network's, in its order.
 __device__ __forceinline__ void sort_vertices(Psa& P) {
     uint32_t n = P.vc;
-    if (n == 3) {
-        cas(P, 1, 2);
-    } else if (n == 4) {
-        cas(P, 1, 3);
-    } else if (n == 5) {
-        cas(P, 2, 4); cas(P, 1, 3); cas(P, 1, 2); cas(P, 0, 3); cas(P, 3, 4);
-    } else if (n == 6) {
-        cas(P, 3, 5); cas(P, 2, 4); cas(P, 1, 5); cas(P, 0, 4); cas(P, 4, 5); cas(P, 1, 3);
-    } else if (n == 7) {
-        cas(P, 2, 5); cas(P, 1, 6); cas(P, 5, 6); cas(P, 3, 4); cas(P, 0, 4); cas(P, 4, 6);
-        cas(P, 1, 3); cas(P, 3, 5); cas(P, 4, 5);
-    } else if (n == 8) {
-        cas(P, 2, 6); cas(P, 3, 7); cas(P, 1, 5); cas(P, 0, 4); cas(P, 4, 6); cas(P, 5, 7);
-        cas(P, 6, 7); cas(P, 4, 5); cas(P, 1, 3);
-    } else if (n == 9) {
+    const bool is3 = n == 3u, is4 = n == 4u, is5 = n == 5u, is6 = n == 6u, is7 = n == 7u, is8 = n == 8u;
+    if (is4 || is5) cas(P, 1, 3);
+    if (is5) cas(P, 0, 3);
+    if (is7) cas(P, 1, 6);
+    if (is5 || is6) cas(P, 2, 4);
+    if (is3 || is5) cas(P, 1, 2);
+    if (is7) cas(P, 2, 5);
+    if (is8) cas(P, 2, 6);
+    if (is5 || is7) cas(P, 3, 4);
+    if (is6 || is7 || is8) cas(P, 0, 4);
+    if (is7) cas(P, 1, 3);
+    if (is8) cas(P, 3, 7);
+    if (is7) cas(P, 5, 6);
+    if (is6 || is7) cas(P, 3, 5);
+    if (is6 || is8) cas(P, 1, 5);
+    if (is6 || is8) cas(P, 1, 3);
+    if (is7 || is8) cas(P, 4, 6);
+    if (is8) cas(P, 5, 7);
+    if (is6 || is7 || is8) cas(P, 4, 5);
+    if (is8) cas(P, 6, 7);
+    if (n == 9u) {
         cas(P, 0, 1); cas(P, 3, 4); cas(P, 6, 7); cas(P, 1, 2); cas(P, 4, 5); cas(P, 7, 8);
         cas(P, 0, 1); cas(P, 3, 4); cas(P, 6, 7); cas(P, 0, 3); cas(P, 3, 6); cas(P, 0, 3);
         cas(P, 1, 4); cas(P, 4, 7); cas(P, 1, 4); cas(P, 2, 5); cas(P, 5, 8); cas(P, 2, 5);
