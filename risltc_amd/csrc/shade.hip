@@ -1253,6 +1253,11 @@ __device__ __forceinline__ bool culled(const Cull& k, float4 s) {
     return hd < -k.dm && hc < -k.cm;
 }
 
+// the shading-space half of culled(): the polygon is below the horizon
+__device__ __forceinline__ bool below_horizon(const Cull& k, float4 s) {
+    return fma_(k.dn, s.w, fma_(k.dz, s.z, fma_(k.dy, s.y, fma_(k.dx, s.x, k.dw)))) < -k.dm;
+}
+
 // The noise LCG advanced by d steps (d < 128) in one affine step: d steps
 // take s to A_d * s + C_d, with A_0 = 1, C_0 = 0, A_{d+1} = a * A_d and
 // C_{d+1} = a * C_d + c. The 128 pairs are a constant table (1 KiB).
@@ -2000,6 +2005,12 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) s
 // rules out the compacted evaluation of shade_kernel. Lights are read from
 // global memory (they stay in L2). The kernel writes the same sample records
 // and compacted shadow rays as shade_kernel, so trace and resolve are shared.
+// A projected-solid-angle candidate below the horizon draws nothing and has
+// target 0: a lane passes over those by their bounding spheres, so the wave
+// evaluates polygons with every lane that still has one (a third of the
+// candidates on the city). One wave per work-group: a wave's time depends on
+// its pixels, and three others would hold its place. Two waves per SIMD; three
+// or four spill (2.13 ms against 2.46 and 2.39 at 640x360, M = 32, 2 spp).
 
 // sample_area_polygon_turk (polygon_sampling_related_work.glsl:34-43): a
 // uniform point on the triangle of vertices 0, 1, 2 (the reference samples
@@ -2065,12 +2076,14 @@ __device__ __forceinline__ void final_turk(const ShadeArgs& A, const Pixel& px, 
 }
 
 template <bool X, uint32_t TECH>
-__global__ void __launch_bounds__(256) shade_baseline_kernel(ShadeArgs A) {
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) shade_baseline_kernel(ShadeArgs A) {
+    // the sample code's column of LDS (clip_materialize)
+    __shared__ float cols[TECH == RISLTC_SAMPLE_POLYGON_PROJECTED_SOLID_ANGLE ? 24 * 64 : 64];
+    float* col_lds = cols + threadIdx.x;
     const uint32_t W = A.c.viewport_size[0], H = A.c.viewport_size[1];
     const uint32_t ww_log2 = A.tile_w_log2, ww = 1u << ww_log2, wh = 64u >> ww_log2;
     const uint32_t tiles_x = (W + ww - 1u) >> ww_log2;
-    const uint32_t tile = blockIdx.x;
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const uint32_t tile = blockIdx.x >> 2, lane = threadIdx.x, wave = blockIdx.x & 3u;
     const uint32_t x = (tile % tiles_x) * ww + (lane & (ww - 1u));
     const uint32_t y = (tile / tiles_x) * (4u * wh) + wave * wh + (lane >> ww_log2);
     const bool inside = x < W && y < H;
@@ -2091,6 +2104,7 @@ __global__ void __launch_bounds__(256) shade_baseline_kernel(ShadeArgs A) {
         seed = murmur_finalize(murmur_mix(murmur_mix(0u, x + y * W), A.c.noise_random_numbers[0]));
     }
     const uint32_t ckey = (shade && A.cache.counts) ? cache_key(A.cache, px.pos, px.n) : 0u;
+    const Cull cull = make_cull(px, A.scene.sphere_bound);
     for (uint32_t j = 0; j < spp; ++j) {
         int32_t chosen = -1;
         float w_sum = 0.0f, sample_value = 0.0f;
@@ -2101,6 +2115,20 @@ __global__ void __launch_bounds__(256) shade_baseline_kernel(ShadeArgs A) {
         } else if (shade) {
             for (uint32_t i = 0; i < M; ++i) {
                 uint32_t idx = light_index_from(noise_next(seed), N);
+                if constexpr (TECH == RISLTC_SAMPLE_POLYGON_PROJECTED_SOLID_ANGLE) {
+                    // a light below the horizon: no draws, target 0
+                    while (i < M && below_horizon(cull, A.scene.spheres[idx])) {
+                        (void)noise_next(seed);
+                        if (A.debug_cands) {
+                            uint32_t* cr = A.debug_cands +
+                                           (((size_t)pixel * spp + j) * M + i) * RISLTC_CANDIDATE_RECORD_WORDS;
+                            cr[0] = idx;
+                            cr[1] = cr[2] = cr[3] = 0u;
+                        }
+                        if (++i < M) idx = light_index_from(noise_next(seed), N);
+                    }
+                    if (i >= M) break;
+                }
                 load_light(A.scene.lights, idx, L);
                 f3 col = mk3(0.0f, 0.0f, 0.0f), point = mk3(0.0f, 0.0f, 0.0f);
                 uint32_t cc = 0;
@@ -2123,7 +2151,7 @@ __global__ void __launch_bounds__(256) shade_baseline_kernel(ShadeArgs A) {
                     // the horizon keeps its unshadowed estimate
                     for (uint32_t it = 0; it < A.iters; ++it) {
                         FinalOut F;
-                        eval_peters<X>(A, px, L, seed, F);
+                        eval_peters<X, true>(A, px, L, seed, F, col_lds);
 #pragma unroll
                         for (int t = 0; t < 2; ++t)
                             if (F.state[t] != 0u) col = add3(col, F.state[t] >= 4u ? F.e_vis[t] : F.e_occ[t]);
@@ -2180,7 +2208,7 @@ __global__ void __launch_bounds__(256) shade_baseline_kernel(ShadeArgs A) {
                     // first shadow ray answers for all of them
                     if (A.light_sampling != RISLTC_LIGHT_UNIFORM && it > 0u && F.state[0] == 5u) F.state[0] = 4u;
                 } else {
-                    eval_peters<X>(A, px, L, seed, F);
+                    eval_peters<X, true>(A, px, L, seed, F, col_lds);
                 }
             }
             put_final<false>(A, lane, inside, contributes, F, px.pos, sidx * A.iters + it, Wt, joint, chosen, ckey);
@@ -2492,7 +2520,8 @@ hipError_t launch_shade(const ShadeArgs& a, bool exact, hipStream_t s) {
 hipError_t launch_shade_baseline(const ShadeArgs& a, uint32_t technique, bool exact, hipStream_t s) {
     // (the baseline kernels write full records only)
     if (!shade_args_ok(a) || a.rec_words != (uint32_t)kSampleWords) return hipErrorInvalidValue;
-    dim3 grid(shade_tiles(a)), block(256);
+    // a wave of its tile per work-group
+    dim3 grid(4u * shade_tiles(a)), block(64);
     if (technique == RISLTC_SAMPLE_POLYGON_AREA_TURK) {
         if (exact) hipLaunchKernelGGL((shade_baseline_kernel<true, RISLTC_SAMPLE_POLYGON_AREA_TURK>), grid, block, 0, s, a);
         else hipLaunchKernelGGL((shade_baseline_kernel<false, RISLTC_SAMPLE_POLYGON_AREA_TURK>), grid, block, 0, s, a);
