@@ -161,130 +161,184 @@ constexpr int kLdW1 = kMlpIn + 8;  // bf16 row strides (16-byte multiples)
 template <int HID>
 constexpr int ld_h() { return HID + 8; }
 
-// LDS of the inference kernel. Width 64: all weights, 8 waves (135 KB).
-// Width 128: the hidden layers' weights (96 KB) and 4 waves; the output
-// layer's weights (64 KB) are read from global memory, where they stay in L2.
-template <int HID, int OUT, int WAVES, bool W4LDS>
+// What bounds it: VALU issue (71% of the cycles at 1080p) on the logits, whose
+// matrix products take a quarter of that time beside it. So the logits' own
+// work is kept small: an insertion into a best-4 in 15 instructions, and for
+// 256 outputs only where a group of four can matter. The weights are not in LDS
+// (135 KB of it for the narrow network, and one wave per SIMD for the wide
+// ones; a view of 62 thousand pixels spent a quarter of its time filling it):
+// they are loaded from L2 as MFMA fragments, each once for a wave's 64 pixels.
+// LDS holds a region per wave, two waves per SIMD for every network: in turn the
+// 64 pixels' features, their hidden activations (a layer reads all its inputs
+// into registers, then writes over them) and, with 256 outputs, the logits of
+// 16 pixels. At 1920x1080, before and after: 128 wide with 1024 outputs 2810
+// and 1381 us, with 256 outputs 1460 and 767, 64 wide with 1024 1369 and 1028,
+// with 256 614 and 468; 333x187 with the last 43 and 28 us. Three waves per SIMD
+// spill (64 wide, 256 outputs: 651 us); chunks of 16 tiles instead of 8 take
+// 447 us there but 34 at 333x187, and chunks of 8 instead of 4 with 128 wide
+// 980 us.
+constexpr int kPropWaves = 4;
+constexpr int kLdX = kMlpIn;  // bf16 row stride of the features, read only once
+template <int HID, int OUT>
 struct PropShared {
-    uint16_t w1[HID * kLdW1];
-    uint16_t w2[HID * ld_h<HID>()];
-    uint16_t w3[HID * ld_h<HID>()];
-    uint16_t w4[W4LDS ? OUT * ld_h<HID>() : 8];
+    static constexpr int kChunk = 512 / HID;      // output tiles at a time (256 outputs)
+    static constexpr int kLdZ = 16 * kChunk + 4;  // floats per pixel of their logits
+    static constexpr int kActBytes = 2 * 64 * (kLdX > ld_h<HID>() ? kLdX : ld_h<HID>());
+    static constexpr int kLogitBytes = OUT > 256 ? 0 : 4 * 16 * kLdZ;
     float bias[3 * HID + OUT];
-    uint32_t csize[OUT];
-    uint16_t act_in[WAVES][16 * kLdW1];
-    uint16_t act_h[WAVES][2][16 * ld_h<HID>()];
+    uint32_t live[OUT];  // all ones, or 0 for an empty cluster
+    uint4 region[kPropWaves][(kActBytes > kLogitBytes ? kActBytes : kLogitBytes) / 16];
 };
-static_assert(sizeof(PropShared<64, 256, 8, true>) <= 160 * 1024, "width-64 LDS");
-static_assert(sizeof(PropShared<128, 256, 4, false>) <= 160 * 1024, "width-128 LDS");
-static_assert(sizeof(PropShared<64, 1024, 8, false>) <= 160 * 1024, "width-64, 1024 outputs LDS");
-static_assert(sizeof(PropShared<128, 1024, 4, false>) <= 160 * 1024, "width-128, 1024 outputs LDS");
+static_assert(sizeof(PropShared<64, 256>) <= 80 * 1024 && sizeof(PropShared<128, 256>) <= 80 * 1024 &&
+                  sizeof(PropShared<64, 1024>) <= 80 * 1024 && sizeof(PropShared<128, 1024>) <= 80 * 1024,
+              "two work-groups per CU");
 
-// one output tile's logits z[i] of clusters c0 + i (i = 0..3) for one pixel:
-// written to `logits` (when not null) and merged into the sorted best-4 bv/bi
-// of the live clusters, in order of i (ties keep the smaller id). Dead
-// clusters read as -inf, and the tile is skipped when its largest logit does
-// not beat the fourth best, which leaves the same best-4 as testing each.
-__device__ __forceinline__ void merge_top4(const float (&z)[4], const bool (&live)[4], int c0, float* logits,
-                                           float (&bv)[4], int (&bi)[4]) {
-    if (logits) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) logits[i] = z[i];
-    }
-    float zc[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) zc[i] = live[i] ? z[i] : -__builtin_inff();
-    if (!(fmax_(fmax_(zc[0], zc[1]), fmax_(zc[2], zc[3])) > bv[3])) return;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        if (zc[i] > bv[3]) {
-            bv[3] = zc[i];
-            bi[3] = c0 + i;
-#pragma unroll
-            for (int q = 3; q > 0; --q)
-                if (bv[q] > bv[q - 1]) {
-                    float tv = bv[q];
-                    bv[q] = bv[q - 1];
-                    bv[q - 1] = tv;
-                    int ti = bi[q];
-                    bi[q] = bi[q - 1];
-                    bi[q - 1] = ti;
-                }
-        }
-    }
+// inserts value v of id into the sorted best-4 (ties keep the earlier one, a
+// NaN is not taken): a sorted list's new entry q is the middle one of v, its
+// old entry and the one before
+__device__ __forceinline__ void insert4(float v, int id, float (&bv)[4], int (&bi)[4]) {
+    const float v0 = bv[0], v1 = bv[1], v2 = bv[2], v3 = bv[3];
+    const int i0 = bi[0], i1 = bi[1], i2 = bi[2], i3 = bi[3];
+    const int n0 = v > v0 ? id : i0, n1 = v > v1 ? id : i1, n2 = v > v2 ? id : i2, n3 = v > v3 ? id : i3;
+    bv[0] = fmax_(v, v0);
+    bv[1] = __builtin_amdgcn_fmed3f(v, v0, v1);
+    bv[2] = __builtin_amdgcn_fmed3f(v, v1, v2);
+    bv[3] = __builtin_amdgcn_fmed3f(v, v2, v3);
+    bi[0] = n0;
+    bi[1] = v > v0 ? i0 : n1;
+    bi[2] = v > v1 ? i1 : n2;
+    bi[3] = v > v2 ? i2 : n3;
 }
 
-// The same for a network of more than 256 outputs, whose table slots name
-// quads of clusters: the tile's four logits are the quad c0 / 4 of this
-// lane, merged as one value, log sum exp over its live clusters (-inf when
-// none is live). Ties keep the smaller quad.
-__device__ __forceinline__ void merge_quad(const float (&z)[4], const bool (&live)[4], int c0, float* logits,
-                                           float (&bv)[4], int (&bi)[4]) {
-    if (logits) {
+// the logit where `live` is all ones, -inf where it is 0 (one v_bfi)
+__device__ __forceinline__ float live_logit(float z, uint32_t live) {
+    return __uint_as_float((__float_as_uint(z) & live) | (0xff800000u & ~live));
+}
+// Four floats or eight halfwords at an address that need only be a multiple of
+// four: the callers' logits and features.
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+
+// max of two that passes one over a NaN, without the quieting of the operands
+// that fmaxf needs for values from bit operations
+__device__ __forceinline__ float max2(float a, float b) { return __builtin_amdgcn_fmed3f(a, b, __builtin_inff()); }
+
+// log sum exp of a quad's logits (-inf: not live); NaN when none is live,
+// which insert4 never takes. The sum is 1 to 4 (or NaN), so its logarithm
+// needs neither the scaling of denormals nor the test for infinity that
+// __logf makes around the same product of log2 and ln 2 (in two parts): 46
+// instead of 53 instructions, the same bits for every float of that range.
+__device__ __forceinline__ float quad_value(const float (&z)[4]) {
+    const float m = fmax_(fmax_(z[0], z[1]), max2(z[2], z[3]));
+    float sum = __expf(z[0] - m);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) logits[i] = z[i];
-    }
-    float m = -__builtin_inff();
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-        if (live[i]) m = fmax_(m, z[i]);
-    if (!(m > -__builtin_inff())) return;
-    float sum = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-        if (live[i]) sum += __expf(z[i] - m);
-    const float v = m + __logf(sum);
-    if (!(v > bv[3])) return;
-    bv[3] = v;
-    bi[3] = c0 >> 2;
-#pragma unroll
-    for (int q = 3; q > 0; --q)
-        if (bv[q] > bv[q - 1]) {
-            float tv = bv[q];
-            bv[q] = bv[q - 1];
-            bv[q - 1] = tv;
-            int ti = bi[q];
-            bi[q] = bi[q - 1];
-            bi[q - 1] = ti;
-        }
+    for (int i = 1; i < 4; ++i) sum += __expf(z[i] - m);
+    const float l = __builtin_amdgcn_logf(sum), hi = l * 0x1.62e42ep-1f;
+    const float lo = fma_(l, 0x1.efa39ep-25f, fma_(l, 0x1.62e42ep-1f, -hi));
+    return m + (hi + lo);
 }
 
-// hidden layer on a 16-pixel tile: out[pixel][o] = relu(W[o] . act[pixel] + b[o])
-template <int HID, int K, int LDW, int LDA>
-__device__ __forceinline__ void hidden_layer(const uint16_t* W, const float* bias, const uint16_t* act, uint16_t* out,
-                                             int lane) {
+// the larger four of two descending lists, descending (values only)
+__device__ __forceinline__ void keep4(float (&a)[4], const float (&b)[4]) {
+    float t[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) t[i] = fmax_(a[i], b[3 - i]);
+    const float p = fmax_(t[0], t[2]), q = fmin_(t[0], t[2]), r = fmax_(t[1], t[3]), s = fmin_(t[1], t[3]);
+    a[0] = fmax_(p, r);
+    a[1] = fmin_(p, r);
+    a[2] = fmax_(q, s);
+    a[3] = fmin_(q, s);
+}
+__device__ __forceinline__ void sort4(float (&a)[4]) {
+    const float p = fmax_(a[0], a[1]), q = fmin_(a[0], a[1]), r = fmax_(a[2], a[3]), s = fmin_(a[2], a[3]);
+    const float u = fmin_(p, r), v = fmax_(q, s);
+    a[0] = fmax_(p, r);
+    a[1] = fmax_(u, v);
+    a[2] = fmin_(u, v);
+    a[3] = fmin_(q, s);
+}
+
+// a layer's weight fragments of output tile t: rows 16 t + r of [out][K]
+template <int K>
+__device__ __forceinline__ void weight_frags(const uint16_t* W, int t, int lane, bf16x8 (&w)[K / 32]) {
+    const uint16_t* p = W + (size_t)(16 * t + (lane & 15)) * K + 8 * (lane >> 4);
+#pragma unroll
+    for (int k = 0; k < K / 32; ++k) w[k] = frag(p + 32 * k);
+}
+
+// the wave's 64 pixels' activations as B fragments: sub-tile s in b[s]
+template <int K, int LD>
+__device__ __forceinline__ void act_frags(const uint16_t* act, int lane, bf16x8 (&b)[4][K / 32]) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int k = 0; k < K / 32; ++k) b[s][k] = frag(act + (16 * s + (lane & 15)) * LD + 32 * k + 8 * (lane >> 4));
+}
+
+// hidden layer on the wave's 64 pixels, in place:
+// act[pixel][o] = relu(W[o] . act[pixel] + bias[o])
+template <int HID, int K, int LD>
+__device__ __forceinline__ void hidden_layer(const uint16_t* W, const float* bias, uint16_t* act, int lane) {
     const int g = lane >> 4, r = lane & 15;
+    bf16x8 b[4][K / 32], w[K / 32];
+    weight_frags<K>(W, 0, lane, w);
+    act_frags<K, LD>(act, lane, b);
+    wave_sync();
+#pragma unroll 2
+    for (int t = 0; t < HID / 16; ++t) {
+        bf16x8 next[K / 32];
+        weight_frags<K>(W, t + 1 < HID / 16 ? t + 1 : t, lane, next);
+        const float4 c = *reinterpret_cast<const float4*>(bias + 16 * t + 4 * g);
 #pragma unroll
-    for (int ot = 0; ot < HID / 16; ++ot) {
-        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+        for (int s = 0; s < 4; ++s) {
+            f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int ks = 0; ks < K / 32; ++ks)
-            acc = mfma(frag(W + (ot * 16 + r) * LDW + ks * 32 + 8 * g), frag(act + r * LDA + ks * 32 + 8 * g), acc);
-        float v[4];
+            for (int k = 0; k < K / 32; ++k) acc = mfma(w[k], b[s][k], acc);
+            const float v[4] = {fmax_(acc[0] + c.x, 0.0f), fmax_(acc[1] + c.y, 0.0f), fmax_(acc[2] + c.z, 0.0f),
+                                fmax_(acc[3] + c.w, 0.0f)};
+            *reinterpret_cast<uint2*>(act + (16 * s + r) * ld_h<HID>() + 16 * t + 4 * g) =
+                make_uint2(bf16_pack2(v[0], v[1]), bf16_pack2(v[2], v[3]));
+        }
 #pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = fmax_(acc[i] + bias[ot * 16 + 4 * g + i], 0.0f);
-        *reinterpret_cast<uint2*>(out + r * ld_h<HID>() + ot * 16 + 4 * g) =
-            make_uint2(bf16_pack2(v[0], v[1]), bf16_pack2(v[2], v[3]));
+        for (int k = 0; k < K / 32; ++k) w[k] = next[k];
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    wave_sync();
+}
+
+// the four table slots of lane group g of a pixel: ids and weights
+// round(255 exp(value - the pixel's largest value))
+__device__ __forceinline__ void put_slots(uint8_t* table, int g, bool in, bool shaded, const float (&bv)[4],
+                                          const int (&bi)[4]) {
+    // the pixel's maximum over its four lanes (lanes r, r+16, r+32, r+48)
+    float zmax = bv[0];
+    zmax = fmax_(zmax, __shfl_xor(zmax, 16));
+    zmax = fmax_(zmax, __shfl_xor(zmax, 32));
+    uint32_t ws = 0, ids = 0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const float e = __expf(bv[q] - zmax) * 255.0f + 0.5f;
+        const uint32_t we = e >= 255.0f ? 255u : (uint32_t)fmax_(e, 0.0f);
+        const uint32_t w = shaded && bv[q] > -__builtin_inff() ? we : 0u;
+        ids |= (w == 0u ? 0u : (uint32_t)bi[q]) << (8 * q);
+        ws |= w << (8 * q);
+    }
+    if (in) {
+        // slot 4 g + q: id at byte 4 g + q, weight at 16 + 4 g + q
+        uint32_t* o = reinterpret_cast<uint32_t*>(table);
+        o[g] = ids;
+        o[4 + g] = ws;
     }
 }
 
-template <int HID, int OUT, int WAVES, bool W4LDS>
-__global__ void __launch_bounds__(64 * WAVES) proposal_kernel(ProposalArgs A) {
-    constexpr int kLdH = ld_h<HID>();
+template <int HID, int OUT>
+__global__ void __launch_bounds__(64 * kPropWaves) __attribute__((amdgpu_waves_per_eu(2)))
+proposal_kernel(ProposalArgs A) {
     constexpr MlpLayout L = mlp_layout(HID, OUT);
-    __shared__ PropShared<HID, OUT, WAVES, W4LDS> sh;
-    const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    // stage the bf16 weights (padded rows) and biases
-    for (int e = tid; e < HID * kMlpIn; e += blockDim.x) sh.w1[(e / kMlpIn) * kLdW1 + e % kMlpIn] = A.wf[L.pw1 + e];
-    for (int e = tid; e < HID * HID; e += blockDim.x) {
-        sh.w2[(e / HID) * kLdH + e % HID] = A.wf[L.pw2 + e];
-        sh.w3[(e / HID) * kLdH + e % HID] = A.wf[L.pw3 + e];
-    }
-    if constexpr (W4LDS)
-        for (int e = tid; e < OUT * HID; e += blockDim.x) sh.w4[(e / HID) * kLdH + e % HID] = A.wf[L.pw4 + e];
-    // the output layer's weights: [out][in] rows of HID bf16
-    const uint16_t* w4 = W4LDS ? sh.w4 : A.wf + L.pw4;
-    constexpr int kLdW4 = W4LDS ? kLdH : HID;
+    constexpr int KH = HID / 32;
+    using Sh = PropShared<HID, OUT>;
+    __shared__ Sh sh;
+    const int tid = (int)threadIdx.x, wave = tid >> 6;
     for (int e = tid; e < HID; e += blockDim.x) {
         sh.bias[e] = A.params[L.pb1 + e];
         sh.bias[HID + e] = A.params[L.pb2 + e];
@@ -292,21 +346,23 @@ __global__ void __launch_bounds__(64 * WAVES) proposal_kernel(ProposalArgs A) {
     }
     for (int e = tid; e < OUT; e += blockDim.x) {
         sh.bias[3 * HID + e] = A.params[L.pb4 + e];
-        sh.csize[e] = (uint32_t)e < A.cluster_count ? A.cluster_offsets[e + 1] - A.cluster_offsets[e] : 0u;
+        sh.live[e] = (uint32_t)e < A.cluster_count && A.cluster_offsets[e + 1] != A.cluster_offsets[e] ? ~0u : 0u;
     }
     __syncthreads();
-    const int g = lane >> 4, r = lane & 15;
-    uint16_t* act = sh.act_in[wave];
-    uint16_t* h0 = sh.act_h[wave][0];
-    uint16_t* h1 = sh.act_h[wave][1];
-    // a wave takes 64 pixels at a time: every lane encodes the features of
-    // one (packed to bf16 pairs in registers), then the MLP runs on the four
-    // 16-pixel sub-tiles in turn, each staged in LDS by its 16 lanes
+    uint16_t* act = reinterpret_cast<uint16_t*>(sh.region[wave]);
     const uint32_t groups = (A.pixel_count + 63u) / 64u;
-    for (uint32_t grp = blockIdx.x * WAVES + wave; grp < groups; grp += gridDim.x * WAVES) {
+    for (uint32_t grp = blockIdx.x * kPropWaves + wave; grp < groups; grp += gridDim.x * kPropWaves) {
+        // keeps the weights' loads and the lane's addresses inside this loop:
+        // hoisted out of it they would need more registers than there are
+        uint32_t none = 0;
+        int lane = tid & 63;
+        asm volatile("" : "+s"(none), "+v"(lane));
+        const int g = lane >> 4, r = lane & 15;
+        const uint16_t *wf = A.wf + none, *w4 = wf + L.pw4;
+        const float* bias4 = sh.bias + 3 * HID + 4 * g;
+        const uint32_t* live4 = sh.live + 4 * g;
         const uint32_t my_pixel = grp * 64u + (uint32_t)lane;
         const bool my_in = my_pixel < A.pixel_count;
-        uint32_t packed[kMlpIn / 2];
         bool my_shaded;
         {
             float f[kMlpIn];
@@ -316,117 +372,25 @@ __global__ void __launch_bounds__(64 * WAVES) proposal_kernel(ProposalArgs A) {
                 for (int k = 0; k < kMlpIn; ++k) f[k] = 0.0f;
             }
 #pragma unroll
-            for (int k = 0; k < kMlpIn; k += 2) packed[k / 2] = bf16_pack2(f[k], f[k + 1]);
-        }
-        if (A.features && my_in) {
-            uint32_t* fo = reinterpret_cast<uint32_t*>(A.features + (size_t)my_pixel * kMlpIn);
-#pragma unroll
-            for (int k = 0; k < kMlpIn / 2; ++k) fo[k] = packed[k];
-        }
-        if constexpr (W4LDS) {
-            // output weights in LDS: the MLP runs on the four 16-pixel
-            // sub-tiles in turn
-#pragma unroll 1
-            for (int sub = 0; sub < 4; ++sub) {
-                if (g == sub) {
-#pragma unroll
-                    for (int k = 0; k < kMlpIn / 2; k += 4)
-                        *reinterpret_cast<uint4*>(act + r * kLdW1 + 2 * k) =
-                            make_uint4(packed[k], packed[k + 1], packed[k + 2], packed[k + 3]);
-                }
-                const uint32_t pixel = grp * 64u + (uint32_t)(16 * sub + r);
-                const bool in = pixel < A.pixel_count;
-                // every lane of the pixel's column learns whether it is shaded
-                const bool shaded = __shfl(my_shaded ? 1 : 0, 16 * sub + r) != 0;
-                wave_sync();
-                hidden_layer<HID, kMlpIn, kLdW1, kLdW1>(sh.w1, sh.bias, act, h0, lane);
-                wave_sync();
-                hidden_layer<HID, HID, kLdH, kLdH>(sh.w2, sh.bias + HID, h0, h1, lane);
-                wave_sync();
-                hidden_layer<HID, HID, kLdH, kLdH>(sh.w3, sh.bias + 2 * HID, h1, h0, lane);
-                wave_sync();
-                // output layer: this lane keeps logits of clusters 16 t + 4 g + i of pixel r,
-                // and the 4 largest of them
-                float bv[4] = {-__builtin_inff(), -__builtin_inff(), -__builtin_inff(), -__builtin_inff()};
-                int bi[4] = {0, 0, 0, 0};
-#pragma unroll 2
-                for (int t = 0; t < OUT / 16; ++t) {
-                    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-                    for (int ks = 0; ks < HID / 32; ++ks)
-                        acc = mfma(frag(w4 + (t * 16 + r) * kLdW4 + ks * 32 + 8 * g),
-                                   frag(h0 + r * kLdH + ks * 32 + 8 * g), acc);
-                    const int c0 = t * 16 + 4 * g;
-                    float z[4];
-                    bool live[4];
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        z[i] = acc[i] + sh.bias[3 * HID + c0 + i];
-                        live[i] = sh.csize[c0 + i] != 0u;
-                    }
-                    float* lo = A.logits && in ? A.logits + (size_t)pixel * OUT + c0 : nullptr;
-                    if constexpr (OUT > 256) merge_quad(z, live, c0, lo, bv, bi);
-                    else merge_top4(z, live, c0, lo, bv, bi);
-                }
-                // the pixel's maximum over its four lanes (lanes r, r+16, r+32, r+48)
-                float zmax = bv[0];
-                zmax = fmax_(zmax, __shfl_xor(zmax, 16));
-                zmax = fmax_(zmax, __shfl_xor(zmax, 32));
-                uint32_t ws = 0;
-#pragma unroll
-                for (int s = 0; s < 4; ++s) {
-                    uint32_t w = 0;
-                    if (shaded && bv[s] > -__builtin_inff()) {
-                        float e = __expf(bv[s] - zmax) * 255.0f + 0.5f;
-                        w = e >= 255.0f ? 255u : (uint32_t)e;
-                    }
-                    if (w == 0u) bi[s] = 0;
-                    ws |= w << (8 * s);
-                }
-                if (in) {
-                    // slot 4 g + s: id at byte 4 g + s, weight at 16 + 4 g + s
-                    uint32_t* o = reinterpret_cast<uint32_t*>(A.out + (size_t)pixel * kPropBytes);
-                    o[g] = (uint32_t)bi[0] | ((uint32_t)bi[1] << 8) | ((uint32_t)bi[2] << 16) | ((uint32_t)bi[3] << 24);
-                    o[4 + g] = ws;
-                }
-                wave_sync();
+            for (int k = 0; k < kMlpIn; k += 8) {
+                const uint4 p = make_uint4(bf16_pack2(f[k], f[k + 1]), bf16_pack2(f[k + 2], f[k + 3]),
+                                           bf16_pack2(f[k + 4], f[k + 5]), bf16_pack2(f[k + 6], f[k + 7]));
+                *reinterpret_cast<uint4*>(act + lane * kLdX + k) = p;
+                if (A.features && my_in)
+                    *reinterpret_cast<u32x4_any*>(A.features + (size_t)my_pixel * kMlpIn + k) =
+                        u32x4_any{p.x, p.y, p.z, p.w};
             }
-        } else {
-            // hidden layers per 16-pixel sub-tile; the last layer's activations of
-            // the four sub-tiles stay in registers as MFMA B fragments (sub-tile s
-            // in hb[3 - s] after the loop), so that the output layer loads each of
-            // its weight fragments once for all 64 pixels
-            bf16x8 hb[4][HID / 32];
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-#pragma unroll
-                for (int ks = 0; ks < HID / 32; ++ks) hb[q][ks] = bf16x8{};
-#pragma unroll 1
-            for (int sub = 0; sub < 4; ++sub) {
-                if (g == sub) {
-#pragma unroll
-                    for (int k = 0; k < kMlpIn / 2; k += 4)
-                        *reinterpret_cast<uint4*>(act + r * kLdW1 + 2 * k) =
-                            make_uint4(packed[k], packed[k + 1], packed[k + 2], packed[k + 3]);
-                }
-                wave_sync();
-                hidden_layer<HID, kMlpIn, kLdW1, kLdW1>(sh.w1, sh.bias, act, h0, lane);
-                wave_sync();
-                hidden_layer<HID, HID, kLdH, kLdH>(sh.w2, sh.bias + HID, h0, h1, lane);
-                wave_sync();
-                hidden_layer<HID, HID, kLdH, kLdH>(sh.w3, sh.bias + 2 * HID, h1, h0, lane);
-                wave_sync();
-#pragma unroll
-                for (int q = 3; q > 0; --q)
-#pragma unroll
-                    for (int ks = 0; ks < HID / 32; ++ks) hb[q][ks] = hb[q - 1][ks];
-#pragma unroll
-                for (int ks = 0; ks < HID / 32; ++ks) hb[0][ks] = frag(h0 + r * kLdH + ks * 32 + 8 * g);
-                // the next sub-tile overwrites act and h0
-                wave_sync();
-            }
-            // output layer: for sub-tile s this lane keeps the logits of clusters
-            // 16 t + 4 g + i of pixel 16 s + r, and the 4 largest of them
+        }
+        wave_sync();
+        hidden_layer<HID, kMlpIn, kLdX>(wf + L.pw1, sh.bias, act, lane);
+        hidden_layer<HID, HID, ld_h<HID>()>(wf + L.pw2, sh.bias + HID, act, lane);
+        hidden_layer<HID, HID, ld_h<HID>()>(wf + L.pw3, sh.bias + 2 * HID, act, lane);
+        bf16x8 hb[4][KH];
+        act_frags<HID, ld_h<HID>()>(act, lane, hb);
+        wave_sync();
+        if constexpr (OUT > 256) {
+            // quads: for sub-tile s this lane ranks quad 4 t + g of pixel
+            // 16 s + r, one value per tile
             float bv[4][4];
             int bi[4][4];
 #pragma unroll
@@ -436,68 +400,143 @@ __global__ void __launch_bounds__(64 * WAVES) proposal_kernel(ProposalArgs A) {
                     bv[s][i] = -__builtin_inff();
                     bi[s][i] = 0;
                 }
-            bf16x8 wa[HID / 32];
-#pragma unroll
-            for (int ks = 0; ks < HID / 32; ++ks) wa[ks] = frag(w4 + r * kLdW4 + ks * 32 + 8 * g);
+            bf16x8 w[KH];
+            weight_frags<HID>(w4, 0, lane, w);
 #pragma unroll 2
             for (int t = 0; t < OUT / 16; ++t) {
-                // the next tile's weight fragments load while this tile's MFMAs run
-                const int tn = t + 1 < OUT / 16 ? t + 1 : t;
-                bf16x8 wn[HID / 32];
+                bf16x8 next[KH];
+                weight_frags<HID>(w4, t + 1 < OUT / 16 ? t + 1 : t, lane, next);
+                const float4 c = *reinterpret_cast<const float4*>(bias4 + 16 * t);
+                const uint4 d = *reinterpret_cast<const uint4*>(live4 + 16 * t);
+                f32x4 z[4];
 #pragma unroll
-                for (int ks = 0; ks < HID / 32; ++ks) wn[ks] = frag(w4 + (tn * 16 + r) * kLdW4 + ks * 32 + 8 * g);
-                float b4[4];
-                bool live[4];
+                for (int s = 0; s < 4; ++s) z[s] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    b4[i] = sh.bias[3 * HID + t * 16 + 4 * g + i];
-                    live[i] = sh.csize[t * 16 + 4 * g + i] != 0u;
+                for (int k = 0; k < KH; ++k)
+#pragma unroll
+                    for (int s = 0; s < 4; ++s) z[s] = mfma(w[k], hb[s][k], z[s]);
+#pragma unroll
+                for (int s = 0; s < 4; ++s) z[s] = f32x4{z[s][0] + c.x, z[s][1] + c.y, z[s][2] + c.z, z[s][3] + c.w};
+                if (A.logits) {
+#pragma unroll
+                    for (int s = 0; s < 4; ++s) {
+                        const uint32_t pixel = grp * 64u + (uint32_t)(16 * s + r);
+                        if (pixel < A.pixel_count)
+                            *reinterpret_cast<f32x4_any*>(A.logits + (size_t)pixel * OUT + 16 * t + 4 * g) = z[s];
+                    }
                 }
 #pragma unroll
                 for (int s = 0; s < 4; ++s) {
-                    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-                    for (int ks = 0; ks < HID / 32; ++ks) acc = mfma(wa[ks], hb[3 - s][ks], acc);
-                    const uint32_t pixel = grp * 64u + (uint32_t)(16 * s + r);
-                    const int c0 = t * 16 + 4 * g;
-                    float z[4];
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) z[i] = acc[i] + b4[i];
-                    float* lo = A.logits && pixel < A.pixel_count ? A.logits + (size_t)pixel * OUT + c0 : nullptr;
-                    if constexpr (OUT > 256) merge_quad(z, live, c0, lo, bv[s], bi[s]);
-                    else merge_top4(z, live, c0, lo, bv[s], bi[s]);
+                    const float zl[4] = {live_logit(z[s][0], d.x), live_logit(z[s][1], d.y), live_logit(z[s][2], d.z),
+                                         live_logit(z[s][3], d.w)};
+                    insert4(quad_value(zl), 4 * t + g, bv[s], bi[s]);
                 }
 #pragma unroll
-                for (int ks = 0; ks < HID / 32; ++ks) wa[ks] = wn[ks];
+                for (int k = 0; k < KH; ++k) w[k] = next[k];
             }
 #pragma unroll
             for (int s = 0; s < 4; ++s) {
                 const uint32_t pixel = grp * 64u + (uint32_t)(16 * s + r);
-                const bool in = pixel < A.pixel_count;
+                const bool shaded = __shfl(my_shaded ? 1 : 0, 16 * s + r) != 0;
+                put_slots(A.out + (size_t)pixel * kPropBytes, g, pixel < A.pixel_count, shaded, bv[s], bi[s]);
+            }
+        } else {
+            // kChunk tiles' weights stay in registers for the four sub-tiles.
+            // Of each the logits go to LDS and the maxima of the lane's
+            // groups of four (one a tile) stay in registers. The best four
+            // logits lie in groups whose maximum is at least the fourth
+            // largest maximum (four others are as large), so only those are
+            // inserted one by one: 4 groups instead of 16, unless maxima tie.
+            constexpr int CT = Sh::kChunk;
+            float* zs = reinterpret_cast<float*>(act);
+            float bv[4][4];
+            int bi[4][4];
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    bv[s][i] = -__builtin_inff();
+                    bi[s][i] = 0;
+                }
+#pragma unroll 1
+            for (int t0 = 0; t0 < OUT / 16; t0 += CT) {
+                bf16x8 w[CT][KH];
+#pragma unroll
+                for (int t = 0; t < CT; ++t) weight_frags<HID>(w4, t0 + t, lane, w[t]);
+#pragma unroll
+                for (int s = 0; s < 4; ++s) {
+                    const uint32_t pixel = grp * 64u + (uint32_t)(16 * s + r);
+                    const bool in = pixel < A.pixel_count;
+                    float top[CT];
+                    uint32_t none4 = 0;  // as above, for the biases
+                    asm volatile("" : "+s"(none4));
+                    const float* bias4s = bias4 + none4;
+                    const uint32_t* live4s = live4 + none4;
+#pragma unroll
+                    for (int t4 = 0; t4 < CT; t4 += 4) {
+                        f32x4 z[4];
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) z[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                        for (int k = 0; k < KH; ++k)
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) z[i] = mfma(w[t4 + i][k], hb[s][k], z[i]);
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const float4 c = *reinterpret_cast<const float4*>(bias4s + 16 * (t0 + t4 + i));
+                            z[i] = f32x4{z[i][0] + c.x, z[i][1] + c.y, z[i][2] + c.z, z[i][3] + c.w};
+                        }
+                        if (A.logits) {
+                            if (in) {
+#pragma unroll
+                                for (int i = 0; i < 4; ++i)
+                                    *reinterpret_cast<f32x4_any*>(A.logits + (size_t)pixel * OUT + 16 * (t0 + t4 + i) + 4 * g) =
+                                        z[i];
+                            }
+                        }
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const int t = t4 + i;
+                            const uint4 d = *reinterpret_cast<const uint4*>(live4s + 16 * (t0 + t));
+                            const float4 zl = make_float4(live_logit(z[i][0], d.x), live_logit(z[i][1], d.y),
+                                                          live_logit(z[i][2], d.z), live_logit(z[i][3], d.w));
+                            *reinterpret_cast<float4*>(zs + r * Sh::kLdZ + 16 * t + 4 * g) = zl;
+                            // -inf for four NaN
+                            top[t] = fmax_(fmax_(zl.x, max2(zl.z, zl.w)), fmax_(zl.y, -__builtin_inff()));
+                        }
+                    }
+                    float best[4] = {top[0], top[1], top[2], top[3]};
+                    sort4(best);
+#pragma unroll
+                    for (int q = 4; q < CT; q += 4) {
+                        float more[4] = {top[q], top[q + 1], top[q + 2], top[q + 3]};
+                        sort4(more);
+                        keep4(best, more);
+                    }
+                    uint32_t groups_of = 0;
+#pragma unroll
+                    for (int t = 0; t < CT; ++t)
+                        groups_of |= (top[t] >= best[3] && top[t] > bv[s][3]) ? 1u << t : 0u;
+                    wave_sync();
+                    while (groups_of != 0u) {
+                        const int t = __builtin_ctz(groups_of);
+                        groups_of &= groups_of - 1u;
+                        const int c0 = 16 * (t0 + t) + 4 * g;
+                        const float4 z = *reinterpret_cast<const float4*>(zs + r * Sh::kLdZ + 16 * t + 4 * g);
+                        insert4(z.x, c0, bv[s], bi[s]);
+                        insert4(z.y, c0 + 1, bv[s], bi[s]);
+                        insert4(z.z, c0 + 2, bv[s], bi[s]);
+                        insert4(z.w, c0 + 3, bv[s], bi[s]);
+                    }
+                    wave_sync();
+                }
+            }
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                const uint32_t pixel = grp * 64u + (uint32_t)(16 * s + r);
                 // every lane of the pixel's column learns whether it is shaded
                 const bool shaded = __shfl(my_shaded ? 1 : 0, 16 * s + r) != 0;
-                // the pixel's maximum over its four lanes (lanes r, r+16, r+32, r+48)
-                float zmax = bv[s][0];
-                zmax = fmax_(zmax, __shfl_xor(zmax, 16));
-                zmax = fmax_(zmax, __shfl_xor(zmax, 32));
-                uint32_t ws = 0;
-                int id[4];
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    uint32_t w = 0;
-                    if (shaded && bv[s][q] > -__builtin_inff()) {
-                        float e = __expf(bv[s][q] - zmax) * 255.0f + 0.5f;
-                        w = e >= 255.0f ? 255u : (uint32_t)e;
-                    }
-                    id[q] = w == 0u ? 0 : bi[s][q];
-                    ws |= w << (8 * q);
-                }
-                if (in) {
-                    // slot 4 g + q: id at byte 4 g + q, weight at 16 + 4 g + q
-                    uint32_t* o = reinterpret_cast<uint32_t*>(A.out + (size_t)pixel * kPropBytes);
-                    o[g] = (uint32_t)id[0] | ((uint32_t)id[1] << 8) | ((uint32_t)id[2] << 16) | ((uint32_t)id[3] << 24);
-                    o[4 + g] = ws;
-                }
+                put_slots(A.out + (size_t)pixel * kPropBytes, g, pixel < A.pixel_count, shaded, bv[s], bi[s]);
             }
         }
     }
@@ -510,20 +549,17 @@ hipError_t launch_proposal(const ProposalArgs& a, hipStream_t s) {
     if (e != hipSuccess) return e;
     const bool wide = a.L.hid == kMlpHidWide, many = a.L.out == kMlpOutWide;
     if ((!wide && a.L.hid != kMlpHid) || (!many && a.L.out != kMlpOut)) return hipErrorInvalidValue;
-    const uint32_t waves = wide ? 4u : 8u;
-    uint32_t groups = (a.pixel_count + 63u) / 64u;
-    uint32_t blocks = (groups + waves - 1u) / waves;
-    uint32_t cap = (uint32_t)(cus > 0 ? cus : 1);
+    const uint32_t groups = (a.pixel_count + 63u) / 64u;
+    uint32_t blocks = (groups + kPropWaves - 1u) / kPropWaves;
+    // the waves take 64 pixels at a time; more than fit at once would only
+    // read the biases again
+    const uint32_t cap = 2u * (uint32_t)(cus > 0 ? cus : 1);
     if (blocks > cap) blocks = cap;
-    dim3 grid(blocks), block(64 * waves);
-    if (wide && many)
-        hipLaunchKernelGGL((proposal_kernel<kMlpHidWide, kMlpOutWide, 4, false>), grid, block, 0, s, a);
-    else if (wide)
-        hipLaunchKernelGGL((proposal_kernel<kMlpHidWide, kMlpOut, 4, false>), grid, block, 0, s, a);
-    else if (many)
-        hipLaunchKernelGGL((proposal_kernel<kMlpHid, kMlpOutWide, 8, false>), grid, block, 0, s, a);
-    else
-        hipLaunchKernelGGL((proposal_kernel<kMlpHid, kMlpOut, 8, true>), grid, block, 0, s, a);
+    dim3 grid(blocks), block(64 * kPropWaves);
+    if (wide && many) hipLaunchKernelGGL((proposal_kernel<kMlpHidWide, kMlpOutWide>), grid, block, 0, s, a);
+    else if (wide) hipLaunchKernelGGL((proposal_kernel<kMlpHidWide, kMlpOut>), grid, block, 0, s, a);
+    else if (many) hipLaunchKernelGGL((proposal_kernel<kMlpHid, kMlpOutWide>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((proposal_kernel<kMlpHid, kMlpOut>), grid, block, 0, s, a);
     return hipGetLastError();
 }
 
