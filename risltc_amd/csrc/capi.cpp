@@ -66,15 +66,14 @@ struct SceneSet {
     rl::BvhBuild bvh;
 };
 
-// everything a batch of views writes: per-view descriptors, the hierarchy
-// table of their scenes, samples, the shared shadow-ray list, hits and
-// counters
+// everything a batch of views writes: the plan (per-view descriptors and the
+// hierarchy table of their scenes, laid out by BatchPlan::layout), samples,
+// the shared shadow-ray list, hits and counters
 struct BatchBuffers {
-    DevBuf shade_args, tile_offsets, resolve_args, block_offsets, bvh_table;
+    DevBuf plan;
     DevBuf samples, rays, ray_slots, hits, counter;
     void release() {
-        DevBuf* b[] = {&shade_args, &tile_offsets, &resolve_args, &block_offsets, &bvh_table, &samples, &rays,
-                       &ray_slots, &hits, &counter};
+        DevBuf* b[] = {&plan, &samples, &rays, &ray_slots, &hits, &counter};
         for (DevBuf* x : b) x->release();
     }
 };
@@ -528,8 +527,12 @@ int risltc_create(risltc_context_t** out, int device) {
         delete c;
         return RISLTC_E_HIP;
     }
-    for (auto& e : c->ev)
-        if (hipEventCreate(&e) != hipSuccess) {
+    // The events between the kernels of a frame only take times: without the
+    // fence to the scope of the system (a write-back of the caches each) the
+    // gaps there are 2 us shorter (a 256x256 frame 114 -> 108 us). ev[3], ev[5] and ev[7] end a call and keep it.
+    for (int i = 0; i < 8; ++i)
+        if (hipEventCreateWithFlags(&c->ev[i], i == 3 || i == 5 || i == 7 ? hipEventDefault
+                                                                          : hipEventDisableSystemFence) != hipSuccess) {
             delete c;
             return RISLTC_E_HIP;
         }
@@ -1645,6 +1648,21 @@ struct BatchPlan {
     bool learned = false, cached = false;  // learned views; the visibility cache is refreshed first
     uint32_t group_log2 = 0;                // table slots name groups of 1 << group_log2 clusters
     rl::VisCacheView cache = {};
+    // Offsets of its parts in BatchBuffers::plan. The hierarchy table is last:
+    // those of the others depend on what `fits` compares only.
+    struct Layout {
+        size_t shade, resolve, tile_off, block_off, bvhs;
+    };
+    Layout layout() const {
+        auto after = [](size_t at, size_t bytes) { return (at + bytes + 255u) / 256u * 256u; };
+        Layout l;
+        l.shade = 0;
+        l.resolve = after(l.shade, shade.size() * sizeof(rl::ShadeArgs));
+        l.tile_off = after(l.resolve, resolve.size() * sizeof(rl::ResolveArgs));
+        l.block_off = after(l.tile_off, tile_off.size() * sizeof(uint32_t));
+        l.bvhs = after(l.block_off, block_off.size() * sizeof(uint32_t));
+        return l;
+    }
     // whether a graph captured with plan `o` can run this plan's descriptors
     bool fits(const BatchPlan& o) const {
         return tile_off == o.tile_off && block_off == o.block_off && samples == o.samples && lds <= o.lds &&
@@ -1756,43 +1774,47 @@ static int plan_batch(risltc_context_t* c, const risltc_view_t* views, uint32_t 
     p.tiles = p.tile_off.back();
     p.blocks = p.block_off.back();
     p.bvh_capacity = std::max<size_t>(p.bvhs.size(), 1u + c->scene_sets.size());
-    if (allocate) HIPC(c, B.bvh_table.ensure(p.bvh_capacity * sizeof(rl::BvhView)));
+    if (allocate) HIPC(c, B.plan.ensure(p.layout().bvhs + p.bvh_capacity * sizeof(rl::BvhView)));
     HIPC(c, rl::trace_blocks(&p.trace_blocks));
     return RISLTC_OK;
 }
 
+// One copy: each is a blocking call of about 14 us. A graph updated and launched
+// with sixteen small views took 490 us with five of them and takes 433 with one.
 static int upload_plan(risltc_context_t* c, BatchBuffers& B, const BatchPlan& p) {
-    HIPC(c, B.shade_args.ensure(p.shade.size() * sizeof(rl::ShadeArgs)));
-    HIPC(c, B.resolve_args.ensure(p.resolve.size() * sizeof(rl::ResolveArgs)));
-    HIPC(c, B.tile_offsets.ensure(p.tile_off.size() * sizeof(uint32_t)));
-    HIPC(c, B.block_offsets.ensure(p.block_off.size() * sizeof(uint32_t)));
-    HIPC(c, hipMemcpy(B.shade_args.p, p.shade.data(), p.shade.size() * sizeof(rl::ShadeArgs), hipMemcpyHostToDevice));
-    HIPC(c, hipMemcpy(B.resolve_args.p, p.resolve.data(), p.resolve.size() * sizeof(rl::ResolveArgs),
-                      hipMemcpyHostToDevice));
-    HIPC(c, hipMemcpy(B.tile_offsets.p, p.tile_off.data(), p.tile_off.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
-    HIPC(c, hipMemcpy(B.block_offsets.p, p.block_off.data(), p.block_off.size() * sizeof(uint32_t),
-                      hipMemcpyHostToDevice));
-    HIPC(c, hipMemcpy(B.bvh_table.p, p.bvhs.data(), p.bvhs.size() * sizeof(rl::BvhView), hipMemcpyHostToDevice));
+    const BatchPlan::Layout l = p.layout();
+    std::vector<uint8_t> host(l.bvhs + p.bvhs.size() * sizeof(rl::BvhView));
+    if (host.size() > B.plan.bytes) return fail(c, RISLTC_E_STATE, "a plan larger than its buffer");
+    memcpy(host.data() + l.shade, p.shade.data(), p.shade.size() * sizeof(rl::ShadeArgs));
+    memcpy(host.data() + l.resolve, p.resolve.data(), p.resolve.size() * sizeof(rl::ResolveArgs));
+    memcpy(host.data() + l.tile_off, p.tile_off.data(), p.tile_off.size() * sizeof(uint32_t));
+    memcpy(host.data() + l.block_off, p.block_off.data(), p.block_off.size() * sizeof(uint32_t));
+    memcpy(host.data() + l.bvhs, p.bvhs.data(), p.bvhs.size() * sizeof(rl::BvhView));
+    HIPC(c, hipMemcpy(B.plan.p, host.data(), host.size(), hipMemcpyHostToDevice));
     return RISLTC_OK;
 }
 
 // kernels only (no memset, no host calls): safe under stream capture
 static int launch_plan(risltc_context_t* c, BatchBuffers& B, const BatchPlan& p, hipStream_t st, bool timed) {
     const uint32_t n = (uint32_t)p.shade.size();
+    const BatchPlan::Layout l = p.layout();
+    const uint8_t* plan = B.plan.as<uint8_t>();
     HIPC(c, rl::launch_zero_u32(B.counter.as<uint32_t>(), kCounterWords, st));
     if (timed) HIPC(c, hipEventRecord(c->ev[0], st));
     if (p.cached) HIPC(c, rl::launch_refresh_cache(p.cache, st));
-    HIPC(c, rl::launch_shade_batch(B.shade_args.as<rl::ShadeArgs>(), B.tile_offsets.as<uint32_t>(), n, p.tiles, p.lds,
-                                   p.exact, p.learned ? 1 : 0, p.general, st));
+    HIPC(c, rl::launch_shade_batch(reinterpret_cast<const rl::ShadeArgs*>(plan + l.shade),
+                                   reinterpret_cast<const uint32_t*>(plan + l.tile_off), n, p.tiles, p.lds, p.exact,
+                                   p.learned ? 1 : 0, p.general, st));
     if (timed) HIPC(c, hipEventRecord(c->ev[1], st));
     if (p.shadows)
-        HIPC(c, rl::launch_trace(trace_args(c, B.bvh_table.as<rl::BvhView>(), B.rays.as<rl::ShadowRay>(),
+        HIPC(c, rl::launch_trace(trace_args(c, reinterpret_cast<const rl::BvhView*>(plan + l.bvhs), B.rays.as<rl::ShadowRay>(),
                                             B.ray_slots.as<uint32_t>(), B.counter.as<uint32_t>(),
                                             B.hits.as<uint32_t>(), p.samples * 2),
                                  st, p.trace_blocks));
     if (timed) HIPC(c, hipEventRecord(c->ev[2], st));
-    HIPC(c, rl::launch_resolve_batch(B.resolve_args.as<rl::ResolveArgs>(), B.block_offsets.as<uint32_t>(), n, p.blocks,
-                                     p.grouped, st));
+    HIPC(c, rl::launch_resolve_batch(reinterpret_cast<const rl::ResolveArgs*>(plan + l.resolve),
+                                     reinterpret_cast<const uint32_t*>(plan + l.block_off), n, p.blocks, p.grouped,
+                                     st));
     if (timed) HIPC(c, hipEventRecord(c->ev[3], st));
     return RISLTC_OK;
 }
