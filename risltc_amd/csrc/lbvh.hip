@@ -300,12 +300,12 @@ __global__ void __launch_bounds__(256) wide_level_kernel(uint32_t level, uint32_
             }
             ++used;
         }
-        // the slot visited first is the last: triangles, then large boxes
-        // (they hold the occluder most often)
+        // small boxes first, then large ones, triangles, and empty slots
+        // last: slot 0 is never empty (wide_fill_kernel counts on it)
         float key[4];
 #pragma unroll
         for (int k = 0; k < 4; ++k)
-            key[k] = s[k] < 0 ? -1.0f : (count[s[k]] > 2 ? node_area(box, s[k]) : __builtin_inff());
+            key[k] = s[k] < 0 ? __builtin_inff() : (count[s[k]] > 2 ? fmin_(node_area(box, s[k]), 1.0e38f) : 2.0e38f);
 #pragma unroll
         for (int k = 0; k < 6; ++k) {
             const int i0 = k < 3 ? k : (k < 5 ? k - 3 : 0);
