@@ -20,6 +20,7 @@
 // same box and Moeller-Trumbore tests in the same operation order, so hit and
 // miss flags agree bit for bit.
 #include <algorithm>
+#include <cmath>
 
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
@@ -428,9 +429,21 @@ struct BuildScratch {
 // the walk's stack, and its rays take the binary walk.
 // scratch: wide_scratch_bytes(n).
 // A node of fewer than four slots holds no wide child, so every wide node
-// with children stands for three binary nodes; n / 2 + 1 holds them all.
+// with children stands for three binary nodes; n / 2 + 1 holds them all. This
+// takes areas that compare: a NaN is never opened, and with NaN throughout a
+// tree of halves has up to 2 n / 3 wide nodes. So the boxes have to be
+// wide_range().
 static size_t wide_scratch_bytes(uint32_t n) {
     return (size_t)(n / 2u + 1u) * (2u * sizeof(int4) + sizeof(int)) + (kWideLevels + 2u) * sizeof(uint32_t);
+}
+
+// Whether the mesh's coordinates (21-bit values, dequantised with what the
+// caller gave) are at most 1e18: no area overflows then, and neither do the
+// walk's plane distances. Any other mesh keeps the binary walk.
+static bool wide_range(const float f[3], const float s[3]) {
+    bool ok = true;
+    for (int a = 0; a < 3; ++a) ok = ok && std::fabs(f[a]) * 2097151.0f + std::fabs(s[a]) <= 1.0e18f;
+    return ok;
 }
 
 static hipError_t build_wide(void* scratch, uint32_t n, const int* left, const int* right, const int* parent,
@@ -560,7 +573,7 @@ hipError_t build_bvh(const uint2* d_pos, uint64_t tri_count, const float deq_fac
                        box, tris, d_pos, rec, unit);
     float4* wide = nullptr;
     hipError_t e = hipGetLastError();
-    if (e == hipSuccess && n > 1 && units < kMaxWideUnits)
+    if (e == hipSuccess && n > 1 && units < kMaxWideUnits && wide_range(deq_factor, deq_summand))
         e = build_wide(tris, (uint32_t)n, left, right, parent, count, box, unit, &wide, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     if (e != hipSuccess) {
