@@ -219,17 +219,13 @@ __device__ __forceinline__ float live_logit(float z, uint32_t live) {
 typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
 typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(4)));
 
-// max of two that passes one over a NaN, without the quieting of the operands
-// that fmaxf needs for values from bit operations
-__device__ __forceinline__ float max2(float a, float b) { return __builtin_amdgcn_fmed3f(a, b, __builtin_inff()); }
-
 // log sum exp of a quad's logits (-inf: not live); NaN when none is live,
 // which insert4 never takes. The sum is 1 to 4 (or NaN), so its logarithm
 // needs neither the scaling of denormals nor the test for infinity that
 // __logf makes around the same product of log2 and ln 2 (in two parts): 46
 // instead of 53 instructions, the same bits for every float of that range.
 __device__ __forceinline__ float quad_value(const float (&z)[4]) {
-    const float m = fmax_(fmax_(z[0], z[1]), max2(z[2], z[3]));
+    const float m = fmax_(fmax_(z[0], z[1]), fmax_(z[2], z[3]));
     float sum = __expf(z[0] - m);
 #pragma unroll
     for (int i = 1; i < 4; ++i) sum += __expf(z[i] - m);
@@ -502,7 +498,7 @@ proposal_kernel(ProposalArgs A) {
                                                           live_logit(z[i][2], d.z), live_logit(z[i][3], d.w));
                             *reinterpret_cast<float4*>(zs + r * Sh::kLdZ + 16 * t + 4 * g) = zl;
                             // -inf for four NaN
-                            top[t] = fmax_(fmax_(zl.x, max2(zl.z, zl.w)), fmax_(zl.y, -__builtin_inff()));
+                            top[t] = fmax_(fmax_(zl.x, fmax_(zl.z, zl.w)), fmax_(zl.y, -__builtin_inff()));
                         }
                     }
                     float best[4] = {top[0], top[1], top[2], top[3]};
