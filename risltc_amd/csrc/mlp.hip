@@ -220,18 +220,13 @@ typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
 typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(4)));
 
 // log sum exp of a quad's logits (-inf: not live); NaN when none is live,
-// which insert4 never takes. The sum is 1 to 4 (or NaN), so its logarithm
-// needs neither the scaling of denormals nor the test for infinity that
-// __logf makes around the same product of log2 and ln 2 (in two parts): 46
-// instead of 53 instructions, the same bits for every float of that range.
+// which insert4 never takes
 __device__ __forceinline__ float quad_value(const float (&z)[4]) {
     const float m = fmax_(fmax_(z[0], z[1]), fmax_(z[2], z[3]));
     float sum = __expf(z[0] - m);
 #pragma unroll
     for (int i = 1; i < 4; ++i) sum += __expf(z[i] - m);
-    const float l = __builtin_amdgcn_logf(sum), hi = l * 0x1.62e42ep-1f;
-    const float lo = fma_(l, 0x1.efa39ep-25f, fma_(l, 0x1.62e42ep-1f, -hi));
-    return m + (hi + lo);
+    return m + __logf(sum);
 }
 
 // the larger four of two descending lists, descending (values only)
