@@ -692,8 +692,8 @@ int risltc_shade_batch(risltc_context_t* context, const risltc_view_t* views, ui
  *                stages its cluster tables when they take at most 16 KiB;
  *                with a visibility cache it keeps three work-groups per CU
  *                at lds_lights = 0;
- *   trace_refill 1..64: twice the idle lanes at which a wave of the
- *                persistent shadow-ray kernel fetches new rays. */
+ *   trace_refill 1..64: idle lanes at which a wave of the persistent
+ *                shadow-ray kernel fetches new rays. */
 typedef struct risltc_tuning_s {
     uint32_t wave_width;
     uint32_t cull_chunk;

@@ -118,7 +118,7 @@ struct risltc_context_s {
     // launch shape (autotuned; RISLTC_TRACE_REFILL overrides the refill at create)
     // (1024 spheres: 16 KB of LDS, so three work-groups fit a CU with the
     // pixel area; more cost a work-group per CU)
-    risltc_tuning_t tuning = {16, 32, 1024, 32};
+    risltc_tuning_t tuning = {16, 32, 1024, 16};
     // extra light sets and meshes for batched views (id = index + 1)
     std::vector<LightSet*> light_sets;
     std::vector<SceneSet*> scene_sets;
@@ -1884,7 +1884,7 @@ int risltc_autotune(risltc_context_t* c, const risltc_view_t* views, uint32_t n,
     if (!c) return RISLTC_E_ARG;
     if (repeats == 0 || repeats > 1000) return fail(c, RISLTC_E_ARG, "repeats %u", repeats);
     HIPC(c, hipSetDevice(c->device));
-    const std::vector<uint32_t> space[4] = {{8, 16, 32, 64}, {8, 16, 32}, {0, 512, 1024, 2048}, {16, 24, 32, 40, 48}};
+    const std::vector<uint32_t> space[4] = {{8, 16, 32, 64}, {8, 16, 32}, {0, 512, 1024, 2048}, {8, 12, 16, 20, 24}};
     risltc_tuning_t best = c->tuning;
     auto field = [](risltc_tuning_t& t, int i) -> uint32_t& {
         return i == 0 ? t.wave_width : i == 1 ? t.cull_chunk : i == 2 ? t.lds_lights : t.trace_refill;

@@ -271,7 +271,7 @@ struct TraceArgs {
     uint32_t max_rays;
     uint32_t* hits;     // one word per slot
     uint32_t* queues;   // kTraceQueues * kQueueStride words, zeroed
-    uint32_t refill;    // a wave fetches rays once half this many lanes are idle
+    uint32_t refill;    // a wave fetches rays once this many lanes are idle
 };
 
 struct ResolveArgs {
