@@ -692,15 +692,16 @@ __device__ __forceinline__ uint32_t closest_hit(const BvhView& B, float3 o, floa
 //   * None is added: a triangle that passes ray_tri counts when the ray also
 //     passes ray_box on the triangle's own bounds. Every ancestor's box
 //     contains them, and ray_box is monotone in the box (each operation is
-//     correctly rounded), so the ancestors pass. Otherwise (a ray within
-//     rounding of the bounds' edge, or parallel to an axis) the lane decides
-//     the ray by the binary walk: about one ray in a million.
-// The binary walk also takes the rays that the error bound below does not
-// cover (negative tmin, components beyond 1e18 or NaN, a direction so close
-// to an axis that the bound exceeds 1% of tmax), walks that would overflow
+//     correctly rounded, and 1 / d is finite, so that none is a NaN), so the
+//     ancestors pass. Otherwise (a ray within rounding of the bounds' edge)
+//     the lane decides the ray by the binary walk: about one ray in a million.
+// The binary walk also takes the rays that this and the error bound below do
+// not cover (negative tmin, components beyond 1e18 or NaN, a component of the
+// direction below 1e-20, 0 among them, a direction so close to an axis that
+// the bound exceeds 1% of tmax), walks that would overflow
 // the stack, and hierarchies without wide nodes.
 //
-// The test: with i = 1 / d clamped to 1e20, a plane's distance is
+// The test: with i = 1 / d, a plane's distance is
 // fma(q, step i, fma(origin, i, -o i)) where ray_box takes (b - o) i. The
 // two differ by at most 2^-21 |o i| plus 2^-21 of the distance; the grid's
 // own rounding is inside the planes' quarter step. err is 2^-20 times the
@@ -735,11 +736,6 @@ struct Walk {
     bool hit;
 };
 
-__device__ __forceinline__ float inverse_clamped(float d) {
-    const float i = 1.0f / d;
-    return __builtin_copysignf(fmin_(fabs_(i), 1.0e20f), i);
-}
-
 __device__ __forceinline__ void walk_start(Walk& w, const BvhView& B, float3 o, float3 d, float tmin, float tmax) {
     w.o = o;
     w.d = d;
@@ -749,7 +745,7 @@ __device__ __forceinline__ void walk_start(Walk& w, const BvhView& B, float3 o, 
     w.wide = (const GlobalF4*)B.wide;
     w.end = (int)B.units;
     w.hit = false;
-    w.in = make_float3(inverse_clamped(d.x), inverse_clamped(d.y), inverse_clamped(d.z));
+    w.in = make_float3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
     w.c = make_float3(-(o.x * w.in.x), -(o.y * w.in.y), -(o.z * w.in.z));
     const float err = 0x1p-20f * fmax_(fmax_(fabs_(w.c.x), fabs_(w.c.y)), fabs_(w.c.z));
     w.lo = tmin + err;
@@ -761,7 +757,8 @@ __device__ __forceinline__ void walk_start(Walk& w, const BvhView& B, float3 o, 
     // (written so that a NaN takes the binary walk)
     const float size = fmax_(fmax_(fmax_(fabs_(o.x), fabs_(o.y)), fabs_(o.z)),
                              fmax_(fmax_(fabs_(d.x), fabs_(d.y)), fabs_(d.z)));
-    const bool plain = size <= 1.0e18f && tmin >= 0.0f && !__builtin_isnan(o.x + o.y + o.z + d.x + d.y + d.z) &&
+    const float steep = fmax_(fmax_(fabs_(w.in.x), fabs_(w.in.y)), fabs_(w.in.z));
+    const bool plain = size <= 1.0e18f && steep <= 1.0e20f && tmin >= 0.0f && !__builtin_isnan(o.x + o.y + o.z + d.x + d.y + d.z) &&
                        !(err > 0.01f * tmax);
     w.mode = plain && B.wide != nullptr ? kWalkWide : kWalkBinary;
 }
@@ -821,8 +818,7 @@ __device__ __forceinline__ bool walk_triangle(const Walk& w, float4 a, float4 b,
                                   fmin_(fmin_(a.z, b.z), c.z), 0.0f);
     const float4 hi = make_float4(fmax_(fmax_(a.x, b.x), c.x), fmax_(fmax_(a.y, b.y), c.y),
                                   fmax_(fmax_(a.z, b.z), c.z), 0.0f);
-    const bool bent = w.d.x != 0.0f && w.d.y != 0.0f && w.d.z != 0.0f;
-    sure = bent && ray_box(w.o, inv, lo, hi, w.tmin, w.tmax);
+    sure = ray_box(w.o, inv, lo, hi, w.tmin, w.tmax);
     return true;
 }
 
