@@ -754,12 +754,12 @@ __device__ __forceinline__ void walk_start(Walk& w, const BvhView& B, float3 o, 
     w.ref = 0;
     w.sp = 0;
     w.bot = 0;
-    // (written so that a NaN takes the binary walk)
+    // (written so that a NaN anywhere, tmax among them, takes the binary walk)
     const float size = fmax_(fmax_(fmax_(fabs_(o.x), fabs_(o.y)), fabs_(o.z)),
                              fmax_(fmax_(fabs_(d.x), fabs_(d.y)), fabs_(d.z)));
     const float steep = fmax_(fmax_(fabs_(w.in.x), fabs_(w.in.y)), fabs_(w.in.z));
-    const bool plain = size <= 1.0e18f && steep <= 1.0e20f && tmin >= 0.0f && !__builtin_isnan(o.x + o.y + o.z + d.x + d.y + d.z) &&
-                       !(err > 0.01f * tmax);
+    const bool plain = size <= 1.0e18f && steep <= 1.0e20f && tmin >= 0.0f && err <= 0.01f * tmax &&
+                       !__builtin_isnan(o.x + o.y + o.z + d.x + d.y + d.z);
     w.mode = plain && B.wide != nullptr ? kWalkWide : kWalkBinary;
 }
 
