@@ -673,9 +673,11 @@ __device__ __forceinline__ uint32_t closest_hit(const BvhView& B, float3 o, floa
 // ---- the shadow walk ---------------------------------------------------------------
 // Any hit over the wide nodes, one ray per lane. A step tests the four boxes
 // of a node or one triangle. The wave takes one kind of step at a time,
-// triangles once kLeafLanes lanes wait at one or no lane is at a node: in
-// one step with the boxes, the triangle code (about 60 instructions, needed by
-// one lane in ten) took more issue slots than they did.
+// triangles once a quarter of its walking lanes wait at one: in one step with
+// the boxes, the triangle code (about 60 instructions, needed by one lane in
+// ten) took more issue slots than they did. (With a fixed count of 16 lanes, a
+// triangle in a wave that had fewer walks left waited for all of them: a
+// thousand random rays through 5000 triangles 112 us instead of 78.)
 //
 // What bounds it: the binary walk read 48 bytes per box, 66 boxes per ray of
 // the 1080p city, and was limited by the vector cache (0.9 tag lookups per
@@ -711,7 +713,7 @@ __device__ __forceinline__ uint32_t closest_hit(const BvhView& B, float3 o, floa
 // passes wherever ray_box's does.
 constexpr int kWalkStack = 20;       // entries per lane: 20 KB of LDS per work-group
 constexpr uint32_t kShareLanes = 16; // idle lanes that make a wave without further rays share its walks
-constexpr uint32_t kLeafLanes = 16;  // lanes at a triangle that make the wave test triangles
+constexpr uint32_t kNodesPerLeaf = 3;  // lanes at a node for one at a triangle: fewer, and the wave tests triangles
 enum WalkMode : uint32_t { kWalkDone = 0, kWalkWide = 1, kWalkBinary = 2 };
 
 // makes one lane's LDS writes visible to the other lanes of its wave
@@ -864,9 +866,8 @@ __device__ __forceinline__ void walk_binary_step(Walk& w) {
 // one step of every walking lane of the wave
 __device__ __forceinline__ void walk_step(Walk& w, int* stack) {
     const bool at_leaf = w.mode == kWalkWide && w.ref < 0, at_node = w.mode == kWalkWide && w.ref >= 0;
-    const uint32_t leaves = (uint32_t)__popcll(__ballot(at_leaf));
-    const bool nodes = __ballot(at_node) != 0ull;
-    if (leaves >= kLeafLanes || !nodes) {
+    const uint32_t leaves = (uint32_t)__popcll(__ballot(at_leaf)), nodes = (uint32_t)__popcll(__ballot(at_node));
+    if (kNodesPerLeaf * leaves >= nodes) {
         if (at_leaf) walk_leaf(w, stack);
     } else if (at_node) {
         walk_node(w, stack);
