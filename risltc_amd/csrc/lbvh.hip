@@ -726,7 +726,7 @@ __device__ __forceinline__ void wave_sync() {
 struct Walk {
     float3 o, d;
     float tmin, tmax;
-    float3 in, c;        // a plane's distance: fma(b, in, c)
+    float3 in, c;        // 1 / d; a plane's distance: fma(b, in, c)
     float lo, hi, slack;  // tmin, tmax and twice the error bound, shifted (wide_boxes)
     const GlobalF4* rec;
     const GlobalF4* wide;
@@ -815,12 +815,11 @@ __device__ __forceinline__ void walk_node(Walk& w, int* stack) {
 __device__ __forceinline__ bool walk_triangle(const Walk& w, float4 a, float4 b, float4 c, bool& sure) {
     float t;
     if (!ray_tri(w.o, w.d, a, b, c, w.tmin, w.tmax, t)) return false;
-    const float3 inv = make_float3(1.0f / w.d.x, 1.0f / w.d.y, 1.0f / w.d.z);
     const float4 lo = make_float4(fmin_(fmin_(a.x, b.x), c.x), fmin_(fmin_(a.y, b.y), c.y),
                                   fmin_(fmin_(a.z, b.z), c.z), 0.0f);
     const float4 hi = make_float4(fmax_(fmax_(a.x, b.x), c.x), fmax_(fmax_(a.y, b.y), c.y),
                                   fmax_(fmax_(a.z, b.z), c.z), 0.0f);
-    sure = ray_box(w.o, inv, lo, hi, w.tmin, w.tmax);
+    sure = ray_box(w.o, w.in, lo, hi, w.tmin, w.tmax);
     return true;
 }
 
@@ -854,8 +853,7 @@ __device__ __forceinline__ void walk_binary_step(Walk& w) {
     if (esc < 0) {
         met = ray_tri(w.o, w.d, a, b, c, w.tmin, w.tmax, t);
     } else {
-        const float3 inv = make_float3(1.0f / w.d.x, 1.0f / w.d.y, 1.0f / w.d.z);
-        next = ray_box(w.o, inv, a, b, w.tmin, w.tmax) ? w.ref + 2 : esc;
+        next = ray_box(w.o, w.in, a, b, w.tmin, w.tmax) ? w.ref + 2 : esc;
     }
     w.hit = met;
     w.ref = next;
