@@ -68,7 +68,8 @@ struct SceneView {
 // origin + byte * step), then their references (>= 0: a wide node, node 0 the
 // root; < 0: a triangle record or a pair of them in rec). The words are
 // origin x y z, step x | step y z, low x, high x | low y, high y, low z,
-// high z | references.
+// high z | references. In front of the nodes lie the units in rec of the binary
+// nodes that they stand for, node 0's last.
 struct BvhView {
     const float4* rec;
     const float4* wide;   // null: no wide nodes
@@ -338,6 +339,7 @@ hipError_t launch_fill_u32(uint32_t* p, uint32_t n, uint32_t v, hipStream_t s);
 struct BvhBuild {
     float4* rec = nullptr;
     float4* wide = nullptr;
+    void* wide_memory = nullptr;  // the allocation: the wide nodes' units, then the nodes
     uint32_t units = 0;
     uint32_t leaf_count = 0;
 };
