@@ -882,9 +882,11 @@ __device__ __forceinline__ void walk_step(Walk& w, int* stack) {
     } else if (at_node) {
         walk_node(w, stack);
     }
-    if (__ballot(w.mode == kWalkBinary) != 0ull) {
+    // (a wave whose walks are all binary stays with them for a while)
+    const int runs = leaves + nodes == 0u ? 8 : 1;
+#pragma unroll 1
+    for (int r = 0; r < runs && __ballot(w.mode == kWalkBinary) != 0ull; ++r)
         if (w.mode == kWalkBinary) walk_binary_step(w, stack);
-    }
 }
 
 // The end of a launch waits for its longest walks, one step per load latency.
