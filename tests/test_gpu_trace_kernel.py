@@ -1,7 +1,7 @@
 """The persistent shadow-ray kernel (runs of rays, refills, walks shared by the
 lanes of a draining wave, subtrees of a full stack) against the oracle's binary
 walk, ray by ray: the debug records of frames over meshes on which its walks
-are long, diverge or overflow, from a handful of rays to several per lane."""
+are long, diverge or overflow, from a handful of rays to 40,000."""
 import ctypes as C
 
 import numpy as np
