@@ -183,11 +183,13 @@ template <int HID, int OUT>
 struct PropShared {
     static constexpr int kChunk = 512 / HID;      // output tiles at a time (256 outputs)
     static constexpr int kLdZ = 16 * kChunk + 4;  // floats per pixel of their logits
+    static constexpr int kLdPair = 2 * 16 + 4;    // floats per pixel of two tiles (1024 outputs)
     static constexpr int kActBytes = 2 * 64 * (kLdX > ld_h<HID>() ? kLdX : ld_h<HID>());
     static constexpr int kLogitBytes = OUT > 256 ? 0 : 4 * 16 * kLdZ;
     float bias[3 * HID + OUT];
     uint32_t live[OUT];  // all ones, or 0 for an empty cluster
     uint4 region[kPropWaves][(kActBytes > kLogitBytes ? kActBytes : kLogitBytes) / 16];
+    static_assert(kActBytes >= 4 * 64 * kLdPair, "two tiles of 64 pixels");
 };
 static_assert(sizeof(PropShared<64, 256>) <= 80 * 1024 && sizeof(PropShared<128, 256>) <= 80 * 1024 &&
                   sizeof(PropShared<64, 1024>) <= 80 * 1024 && sizeof(PropShared<128, 1024>) <= 80 * 1024,
@@ -322,7 +324,16 @@ __device__ __forceinline__ void put_slots(uint8_t* table, int g, bool in, bool s
     }
 }
 
-template <int HID, int OUT>
+// LOGITS: whether the caller's logits are written. 1024 of them a pixel are
+// bound by those stores. A lane has four of a tile, so a tile's store is 64
+// bytes at a time, 4 KB apart, and half lines leave L2; and a wait for the next
+// weights waits for the stores before it too. Two tiles therefore go through
+// LDS and out as 128 contiguous bytes a pixel: 1300x777, 128 wide, 2080 -> 1230
+// us (with one tile's ranking between its stores and the next products alone:
+// 2060), 64 wide 1580 -> 1050. Without the logits the kernel is its own
+// instantiation. With 256 outputs the weights of several tiles are loaded at
+// once, the stores cost 80 of 490 us, and one instantiation serves both.
+template <int HID, int OUT, bool LOGITS>
 __global__ void __launch_bounds__(64 * kPropWaves) __attribute__((amdgpu_waves_per_eu(2)))
 proposal_kernel(ProposalArgs A) {
     constexpr MlpLayout L = mlp_layout(HID, OUT);
@@ -408,13 +419,35 @@ proposal_kernel(ProposalArgs A) {
                     for (int s = 0; s < 4; ++s) z[s] = mfma(w[k], hb[s][k], z[s]);
 #pragma unroll
                 for (int s = 0; s < 4; ++s) z[s] = f32x4{z[s][0] + c.x, z[s][1] + c.y, z[s][2] + c.z, z[s][3] + c.w};
-                if (A.logits) {
+                if constexpr (LOGITS) {
+                    float* zs = reinterpret_cast<float*>(act);
 #pragma unroll
-                    for (int s = 0; s < 4; ++s) {
-                        const uint32_t pixel = grp * 64u + (uint32_t)(16 * s + r);
-                        if (pixel < A.pixel_count)
-                            *reinterpret_cast<f32x4_any*>(A.logits + (size_t)pixel * OUT + 16 * t + 4 * g) = z[s];
+                    for (int s = 0; s < 4; ++s)
+                        *reinterpret_cast<f32x4*>(zs + (16 * s + r) * Sh::kLdPair + 16 * (t & 1) + 4 * g) = z[s];
+                    if ((t & 1) != 0) {
+                        wave_sync();
+                        const uint32_t p0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(grp * 64u));
+                        float* out = A.logits + (size_t)p0 * OUT + 16 * (t - 1);
+                        const uint32_t row = (uint32_t)lane >> 3, col = 4u * ((uint32_t)lane & 7u);
+                        auto put = [&](uint32_t j) {
+                            *reinterpret_cast<f32x4_any*>(out + ((row + j) * (uint32_t)OUT + col)) =
+                                *reinterpret_cast<const f32x4*>(zs + (row + j) * Sh::kLdPair + col);
+                        };
+                        // (without the test the eight reads are in flight together)
+                        if (A.pixel_count - p0 >= 64u) {
+#pragma unroll
+                            for (uint32_t j = 0; j < 64u; j += 8u) put(j);
+                        } else {
+#pragma unroll 1
+                            for (uint32_t j = 0; j < 64u; j += 8u)
+                                if (row + j < A.pixel_count - p0) put(j);
+                        }
+                        wave_sync();
                     }
+                } else {
+                    // (a tile's products mixed with its ranking: 1401 us at
+                    // 1920x1080, 128 wide, instead of 1332)
+                    __builtin_amdgcn_sched_barrier(0);
                 }
 #pragma unroll
                 for (int s = 0; s < 4; ++s) {
@@ -547,10 +580,16 @@ hipError_t launch_proposal(const ProposalArgs& a, hipStream_t s) {
     const uint32_t cap = 2u * (uint32_t)(cus > 0 ? cus : 1);
     if (blocks > cap) blocks = cap;
     dim3 grid(blocks), block(64 * kPropWaves);
-    if (wide && many) hipLaunchKernelGGL((proposal_kernel<kMlpHidWide, kMlpOutWide>), grid, block, 0, s, a);
-    else if (wide) hipLaunchKernelGGL((proposal_kernel<kMlpHidWide, kMlpOut>), grid, block, 0, s, a);
-    else if (many) hipLaunchKernelGGL((proposal_kernel<kMlpHid, kMlpOutWide>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((proposal_kernel<kMlpHid, kMlpOut>), grid, block, 0, s, a);
+    if (many && a.logits) {
+        if (wide) hipLaunchKernelGGL((proposal_kernel<kMlpHidWide, kMlpOutWide, true>), grid, block, 0, s, a);
+        else hipLaunchKernelGGL((proposal_kernel<kMlpHid, kMlpOutWide, true>), grid, block, 0, s, a);
+    } else if (many) {
+        if (wide) hipLaunchKernelGGL((proposal_kernel<kMlpHidWide, kMlpOutWide, false>), grid, block, 0, s, a);
+        else hipLaunchKernelGGL((proposal_kernel<kMlpHid, kMlpOutWide, false>), grid, block, 0, s, a);
+    } else {
+        if (wide) hipLaunchKernelGGL((proposal_kernel<kMlpHidWide, kMlpOut, true>), grid, block, 0, s, a);
+        else hipLaunchKernelGGL((proposal_kernel<kMlpHid, kMlpOut, true>), grid, block, 0, s, a);
+    }
     return hipGetLastError();
 }
 
