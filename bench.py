@@ -60,8 +60,10 @@ LEARN_PATH_FRAMES = 200
 LARGE_PATH_FRAMES = 100
 HBM_PEAK_GBS = 8000.0
 # wave64 FP32 VALU instructions: 256 CUs x 4 SIMDs, 4 cycles each, 2.4 GHz
-# (non-packed: the build disables packed FP32), in lane-instructions/s
+# (non-packed: the build disables packed FP32), in lane-instructions/s. An
+# estimate: the shadow-ray kernel issues one in 3.4 cycles, so some take fewer
 VALU_PEAK_TLANE = 256 * 4 * 16 * 2.4e9 / 1e12
+SIMD_CYCLES_PER_MS = 256 * 4 * 2.4e6
 # dense BF16 MFMA peak of the MI355X
 MFMA_BF16_PEAK_TF = 2500.0
 PMC_FILE = os.path.join(ROOT, "profiles", "shade_city1080_traffic.json")
@@ -379,7 +381,7 @@ def kernel_report(kernel_ms, pixels, samples, rays, shade_alg, learned):
         if c:
             r["measured_bytes"] = c["bytes_per_launch"]
             r["measured_hbm_frac"] = round(c["bytes_per_launch"] / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4)
-            r["valu_frac"] = round(c["valu_insts_per_launch"] * 64 / (ms * 1e-3) / 1e12 / VALU_PEAK_TLANE, 4)
+            r["simd_cycles_per_valu_inst"] = round(SIMD_CYCLES_PER_MS * ms / c["valu_insts_per_launch"], 2)
             r["active_lanes"] = round(c["valu_thread_cycles_per_launch"] / c["valu_insts_per_launch"] / 64, 3)
         out[k] = r
     if learned:
@@ -655,7 +657,8 @@ def main():
         roofline["measured_traffic_frac"] = round(measured / HBM_PEAK_GBS, 4)
     if valu:
         roofline["limiter"] = "valu" if valu["frac"] >= roofline.get("measured_traffic_frac", 0.0) else "hbm"
-        roofline["limiter_frac"] = max(valu["frac"], roofline.get("measured_traffic_frac", 0.0))
+        roofline["limiter_frac"] = min(1.0, max(valu["frac"], roofline.get("measured_traffic_frac", 0.0)))
+        roofline["limiter_basis"] = "estimate, 4 cycles per VALU instruction; measured HBM bytes"
     kernels = kernel_report(kernel_ms, P, samples, rays, alg, learned)
     line = {
         "metric": METRIC,

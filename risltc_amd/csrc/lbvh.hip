@@ -684,9 +684,13 @@ __device__ __forceinline__ uint32_t closest_hit(const BvhView& B, float3 o, floa
 // the 1080p city, and was limited by the vector cache (0.9 tag lookups per
 // clock and CU); four-way nodes of float planes (112 bytes) had the same limit
 // (2.2 ms against 1.65). With byte planes a node is four 16-byte loads, and
-// issue and lookups are about level: 1.2 ms for 10.8M rays, 13.9 nodes and 2.2
+// issue and lookups are about level: 1.13 ms for 10.8M rays, 13.9 nodes and 2.2
 // triangles each (83% occluded; without the chord order 17.4 and 2.6), 35 of
-// 64 lanes active at a node. 16,384 lights, 45M rays: 7.7 -> 5.2 ms.
+// 64 lanes active at a node. 16,384 lights, 34.6M rays: 7.7 -> 4.8 ms. A step
+// is about 140 VALU instructions where a binary step is 30, so a wave whose
+// rays are nearly the same, and whose binary records stay in its L1, is slower
+// than it was (1000 rays of one origin within 1e-4 through 200,000 triangles: 50
+// us against 36), and so are rays through triangles piled on each other.
 //
 // The flag is the binary walk's, bit for bit: a ray is occluded when some
 // triangle passes ray_tri and every binary node above it passes ray_box.
@@ -942,11 +946,11 @@ __device__ __forceinline__ bool walk_share(Walk& w, uint32_t& slot, bool shared,
 // in runs: the first from the wave's place in its slice, later ones from
 // the slice's counter. (With one atomic per refill, waves without rays queued
 // at eight counters: 0.1 of the 0.125 ms of a 63k-ray list.)
-// Seven waves per SIMD: 72 VGPRs, no spills (eight spill: 1.8 ms against 1.2).
-// Every wave leaves the loop: a wide walk visits a reference at most once
-// before it ends or turns into a binary walk, which is bounded; each refill
-// takes rays or moves to the next slice, and after kTraceQueues slices there
-// is nothing left to fetch.
+// Seven waves per SIMD: 70 VGPRs, no spills (eight spill: 1.8 ms against 1.2).
+// Every wave leaves the loop: a wide walk only goes down, visiting a node at
+// most once and a triangle at most once per slot that names it, and a binary
+// walk moves forward in pre-order; each refill takes rays or moves to the next
+// slice, and after kTraceQueues slices there is nothing left to fetch.
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) trace_kernel(TraceArgs A) {
     __shared__ int stacks[kWalkStack * 256];
     __shared__ int pair_lanes[256];

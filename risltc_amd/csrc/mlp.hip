@@ -161,8 +161,10 @@ constexpr int kLdW1 = kMlpIn + 8;  // bf16 row strides (16-byte multiples)
 template <int HID>
 constexpr int ld_h() { return HID + 8; }
 
-// What bounds it: VALU issue (71% of the cycles at 1080p) on the logits, whose
-// matrix products take a quarter of that time beside it. So the logits' own
+// What bounds it: VALU work on the logits, beside their matrix products. At
+// 1080p, with four cycles to an instruction, VALU takes 58% of the cycles with
+// 64 wide and 256 outputs and 72% with 128 wide and 1024, MFMA 10% and 22%,
+// and waves wait for a third and a quarter of theirs. So the logits' own
 // work is kept small: an insertion into a best-4 in 15 instructions, and for
 // 256 outputs only where a group of four can matter. The weights are not in LDS
 // (135 KB of it for the narrow network, and one wave per SIMD for the wide
@@ -172,9 +174,11 @@ constexpr int ld_h() { return HID + 8; }
 // 64 pixels' features, their hidden activations (a layer reads all its inputs
 // into registers, then writes over them) and, with 256 outputs, the logits of
 // 16 pixels. At 1920x1080, before and after: 128 wide with 1024 outputs 2810
-// and 1381 us, with 256 outputs 1460 and 767, 64 wide with 1024 1369 and 1028,
-// with 256 614 and 468; 333x187 with the last 43 and 28 us. Three waves per SIMD
-// spill (64 wide, 256 outputs: 651 us); chunks of 16 tiles instead of 8 take
+// and 1332 us, with 256 outputs 1460 and 767, 64 wide with 1024 1369 and 1080,
+// with 256 614 and 466; 333x187 with the last 43 and 28 us. Two waves per SIMD
+// have 256 VGPRs: 256 outputs spill 46 (128 wide) and 30 of them, 1024 outputs
+// 8 or 28 (128 wide, with logits) and none. Three waves per SIMD spill in the
+// inner loops (64 wide, 256 outputs: 651 us); chunks of 16 tiles instead of 8 take
 // 447 us there but 34 at 333x187, and chunks of 8 instead of 4 with 128 wide
 // 980 us.
 constexpr int kPropWaves = 4;
@@ -602,7 +606,7 @@ hipError_t launch_proposal(const ProposalArgs& a, hipStream_t s) {
 // activations and logits in LDS; what leaves it are the transposed
 // activations and gradients, whose rows the weight gradients read K-contiguous.
 // What bounds it: 12 GFLOP on 65,536 rows are 10 us of matrix cores; the 24
-// small launches that this replaces took 830 us (of them 440 in sums by one
+// small launches that this replaces took 730 us (of them 440 in sums by one
 // work-group with one load in flight).
 __device__ __forceinline__ uint32_t hash32(uint32_t x) {
     x ^= x >> 16;

@@ -281,7 +281,8 @@ __device__ __forceinline__ float polygon_ltc(const float* px, const float* py, c
                 a = b;
             }
             r = mask != 0u ? fabs_(acc) : 0.0f;
-            // an edge longer than 90 degrees (or a NaN) takes the general form
+            // an edge longer than 90 degrees takes the general form (one with
+            // a NaN makes the sum NaN in either)
             general = __builtin_amdgcn_ballot_w64(mask != 0u && !(shortest > 0.0f)) != 0ull;
         }
     }
@@ -2001,16 +2002,18 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) s
 // The two polygon sampling techniques the reference compares against
 // (src/experiment_list.c:313-396), with the uniform source. One lane per
 // pixel evaluates its candidates one after the other: a projected-solid-angle
-// candidate consumes 0, 2 or 4 noise draws depending on the polygon, which
-// rules out the compacted evaluation of shade_kernel. Lights are read from
+// candidate consumes 0, 2 or 4 noise draws depending on its polygon, so a
+// candidate's place in the noise follows from the polygons before it, where
+// shade_kernel's compacted evaluation has it from an index. Lights are read from
 // global memory (they stay in L2). The kernel writes the same sample records
 // and compacted shadow rays as shade_kernel, so trace and resolve are shared.
 // A projected-solid-angle candidate below the horizon draws nothing and has
 // target 0: a lane passes over those by their bounding spheres, so the wave
 // evaluates polygons with every lane that still has one (a third of the
 // candidates on the city). One wave per work-group: a wave's time depends on
-// its pixels, and three others would hold its place. Two waves per SIMD; three
-// or four spill (2.13 ms against 2.46 and 2.39 at 640x360, M = 32, 2 spp).
+// its pixels, and three others would hold its place. Two waves per SIMD (256
+// VGPRs, 14 of them spilled, 19 in the exact build); three or four spill more
+// (2.13 ms against 2.46 and 2.39 at 640x360, M = 32, 2 spp).
 
 // sample_area_polygon_turk (polygon_sampling_related_work.glsl:34-43): a
 // uniform point on the triangle of vertices 0, 1, 2 (the reference samples
