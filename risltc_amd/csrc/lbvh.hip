@@ -855,24 +855,27 @@ __device__ __forceinline__ void walk_leaf(Walk& w, const int* stack) {
     w.mode = met ? (sure ? kWalkDone : kWalkBinary) : (more ? kWalkWide : kWalkDone);
 }
 
-// One step of the binary walk. Every step moves forward in pre-order (by 2,
-// by 3 or to an escape unit past the node's subtree), so it ends; reads of a
-// record at unit x < end touch x .. x + 2, inside the padded array. After a
+// Up to `steps` steps of the binary walk. Every step moves forward in pre-order
+// (by 2, by 3 or to an escape unit past the node's subtree), so it ends; reads
+// of a record at unit x < end touch x .. x + 2, inside the padded array. After a
 // subtree without a hit the walk goes on with the stack.
-__device__ __forceinline__ void walk_binary_step(Walk& w, const int* stack) {
-    const float4 a = global_f4(w.rec, w.ref), b = global_f4(w.rec, w.ref + 1), c = global_f4(w.rec, w.ref + 2);
-    const int esc = __float_as_int(a.w);
-    float t;
+__device__ __forceinline__ void walk_binary(Walk& w, const int* stack, int steps) {
+    int x = w.ref;
     bool met = false;
-    int next = w.ref + 3;
-    if (esc < 0) {
-        met = ray_tri(w.o, w.d, a, b, c, w.tmin, w.tmax, t);
-    } else {
-        next = ray_box(w.o, w.in, a, b, w.tmin, w.tmax) ? w.ref + 2 : esc;
-    }
-    const bool over = met || next >= w.end, more = over && !met && w.sp > w.bot;
+    do {
+        const float4 a = global_f4(w.rec, x), b = global_f4(w.rec, x + 1), c = global_f4(w.rec, x + 2);
+        const int esc = __float_as_int(a.w);
+        if (esc < 0) {
+            float t;
+            met = ray_tri(w.o, w.d, a, b, c, w.tmin, w.tmax, t);
+            x += 3;
+        } else {
+            x = ray_box(w.o, w.in, a, b, w.tmin, w.tmax) ? x + 2 : esc;
+        }
+    } while (--steps > 0 && !met && x < w.end);
+    const bool over = met || x >= w.end, more = over && !met && w.sp > w.bot;
     w.hit = met;
-    w.ref = next;
+    w.ref = x;
     if (more) w.ref = stack[--w.sp * 256];
     w.mode = more ? kWalkWide : (over ? kWalkDone : kWalkBinary);
 }
@@ -887,10 +890,10 @@ __device__ __forceinline__ void walk_step(Walk& w, int* stack) {
         walk_node(w, stack);
     }
     // (a wave whose walks are all binary stays with them for a while)
-    const int runs = leaves + nodes == 0u ? 8 : 1;
-#pragma unroll 1
-    for (int r = 0; r < runs && __ballot(w.mode == kWalkBinary) != 0ull; ++r)
-        if (w.mode == kWalkBinary) walk_binary_step(w, stack);
+    if (__ballot(w.mode == kWalkBinary) != 0ull) {
+        const int steps = leaves + nodes == 0u ? 16 : 1;
+        if (w.mode == kWalkBinary) walk_binary(w, stack, steps);
+    }
 }
 
 // The end of a launch waits for its longest walks, one step per load latency.
