@@ -61,7 +61,7 @@ LARGE_PATH_FRAMES = 100
 HBM_PEAK_GBS = 8000.0
 # wave64 FP32 VALU instructions: 256 CUs x 4 SIMDs, 4 cycles each, 2.4 GHz
 # (non-packed: the build disables packed FP32), in lane-instructions/s. An
-# estimate: the shadow-ray kernel issues one in 3.4 cycles, so some take fewer
+# estimate: the shadow-ray kernel issues one in 3.3 cycles, so some take fewer
 VALU_PEAK_TLANE = 256 * 4 * 16 * 2.4e9 / 1e12
 SIMD_CYCLES_PER_MS = 256 * 4 * 2.4e6
 # dense BF16 MFMA peak of the MI355X
